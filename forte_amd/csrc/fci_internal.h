@@ -87,10 +87,11 @@ struct SpinTables {
     // when the excitation does not exist. P = (r,r): J = I when r occupied.
     int np = 0;
     DBuf<uint32_t> out;   // [np * nstr], pair-major
-    // the same targets as 16-bit entries (address | sign << 15, 0x7FFF = none) in the paired-column
-    // MFMA tile layout [ceil(nstr/32)][npp/16][64 lanes][2][4] (npp = np rounded up to 16): the 8
-    // targets of lane (g, c) for strings 32 it + 2c + p and pairs 16 tile + 4 g + v are one 16-byte
-    // word; built only when nstr <= 32767
+    // the same targets as 16-bit entries (slot in the LDS row | sign << 15) in the paired-column MFMA
+    // tile layout [ceil(nstr/32)][npp/16][64 lanes][2][4] (npp = np rounded up to 16): the 8 targets of
+    // lane (g, c) for strings 32 it + 2c + p and pairs 16 tile + 4 g + v are one 16-byte word, and each
+    // string's 4 are one 8-byte word; string J has slot ab_slot(J), and an excitation that does not
+    // exist has one of the 64 unused slots behind the row. Built only when the slots fit in 15 bits.
     int npp = 0;
     DBuf<uint16_t> outT;
     // pair cliques for the same-spin operator: hole strings K with k-d electrons (d = 2, or 1
@@ -104,6 +105,15 @@ struct SpinTables {
     int nown = 0;
     DBuf<uint32_t> own;   // [nstr * nown]
 };
+
+// The row of sigma that an alpha-beta kernel accumulates in LDS: within 32 strings the even ones come
+// first, so that both 16 consecutive strings and every other one of 32 fall into 16 different banks
+// (FP64 LDS atomics of a wave, 4 runs of 16 strings: 8.3 cycles, against 16.2 for every other string of
+// a row in plain order). Behind the strings, 64 slots that absorb what does not exist: without a
+// divergent branch a scattered value takes 5 vector instructions instead of 11, and inactive lanes save
+// an atomic nothing (8.1 cycles with half of them).
+__host__ __device__ inline int ab_slot(int J) { return (J & ~31) | ((J & 1) << 4) | ((J >> 1) & 15); }
+__host__ __device__ inline int64_t ab_row_slots(int64_t nstr) { return (nstr + 31) / 32 * 32 + 64; }
 
 void build_spin_tables(SpinTables& t, int n, int k, const uint32_t* d_binom, hipStream_t st);
 // point-group classes of the strings: irrep (XOR of the occupied orbitals' irreps, orbsym in
@@ -237,6 +247,12 @@ struct BatchSigmaTabs {
 bool batch_sigma_supported(const SpinTables& a, const SpinTables& b, std::string* why);
 // elements of scratch per item; *off_yt and *off_e: offsets of Y^T and E inside it (C^T at 0)
 size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, size_t* off_yt, size_t* off_e);
+// the FP64 alpha-beta term with the gathered rows staged in LDS (fci_ab64.hip): whether it takes these
+// tables, sigma += H_ab C with the packed integrals vpk, the batched form and its kernel attributes
+bool ab5_f64_ok(const SpinTables& a, const SpinTables& b);
+void ab5_f64(const double* C, double* S, const SpinTables& a, const SpinTables& b, const double* vpk, hipStream_t st);
+void ab5_f64_batch(const SpinTables& a, const SpinTables& b, const BatchSigmaTabs& t, hipStream_t st);
+void ab5_f64_prepare(const SpinTables& a, const SpinTables& b);
 // sets the kernel attributes batch_sigma_f64 needs (call before capturing it in a graph)
 void batch_sigma_prepare(const SpinTables& a, const SpinTables& b);
 void batch_sigma_f64(const SpinTables& a, const SpinTables& b, int gd_a, int gd_b, const BatchSigmaTabs& t,

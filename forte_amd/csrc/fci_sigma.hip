@@ -1435,7 +1435,9 @@ __global__ __launch_bounds__(256) void k_ab_mixed(const float* __restrict__ C, f
 // table (8 targets per lane and tile = one 16-byte load; a wave's loads are contiguous).
 // The LDS row accumulates in FP64: on gfx950 an LDS FP64 atomic add of a full wave costs about a
 // seventh of the FP32 one, which is serialized per lane. Requires Nb even and Nb <= 32767.
-constexpr uint16_t kInv16 = 0x7FFFu;
+// a scattered value's slot in the row and its sign: half h (0, 1) of a target word
+__device__ __forceinline__ uint32_t ab_target(uint32_t w, int h) { return h ? (w >> 16) & 0x7FFFu : w & 0x7FFFu; }
+__device__ __forceinline__ uint32_t ab_sign(uint32_t w, int h) { return (h ? w : w << 16) & 0x80000000u; }
 
 template <int KS, int TPW, int WM, int WC>
 __global__ __launch_bounds__(64 * WM * WC) void k_ab2_mixed(const float* __restrict__ C, float* __restrict__ S, int64_t Na,
@@ -1443,7 +1445,7 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab2_mixed(const float* __restr
                                                       const uint32_t* __restrict__ str_a,
                                                       const uint16_t* __restrict__ outT, int npp, int np,
                                                       const float* __restrict__ vpk, int nmt) {
-    extern __shared__ __attribute__((aligned(16))) double srow_m[];  // [Nb]
+    extern __shared__ __attribute__((aligned(16))) double srow_m[];  // [ab_row_slots(Nb)]
     double* srow = srow_m;
     __shared__ uint32_t ent[KS * 32];
     __shared__ float vdg[12 * 16];
@@ -1454,7 +1456,7 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab2_mixed(const float* __restr
     const int wm = wave % WM, wc = wave / WM;
     const int g = lane >> 4, cl = lane & 15;
     for (int i = tid; i < KS * 32; i += NTH) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
-    for (int64_t i = tid; i < Nb; i += NTH) srow[i] = 0.0;
+    for (int i = tid; i < int(ab_row_slots(Nb)); i += NTH) srow[i] = 0.0;
     const uint32_t occ = str_a[Ja];
     for (int r = tid; r < nmt * 16; r += NTH) {  // diagonal excitations: sum_{q in Ja} (qq|r)
         float d = 0.f;
@@ -1541,16 +1543,16 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab2_mixed(const float* __restr
             for (int p = 0; p < 2; ++p)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const uint32_t tt = (tw[p * 2 + v / 2] >> (16 * (v & 1))) & 0xFFFFu;
-                    if (!ok || (tt & 0x7FFFu) == kInv16) continue;
+                    const uint32_t w = tw[p * 2 + v / 2];
                     const float a = (p ? a1[v] : a0[v]) + vd[j][v] * (p ? cd.y : cd.x);
-                    atomicAdd(&srow[tt & 0x7FFFu], double((tt >> 15) ? -a : a));
+                    atomicAdd(&srow[ab_target(w, v & 1)],
+                              double(__uint_as_float(__float_as_uint(a) ^ ab_sign(w, v & 1))));
                 }
         }
     }
     __syncthreads();
     float* Srow = S + Ja * Nb;
-    for (int64_t i = tid; i < Nb; i += NTH) Srow[i] = float(double(Srow[i]) + srow[i]);
+    for (int i = tid; i < int(Nb); i += NTH) Srow[i] = float(double(Srow[i]) + srow[ab_slot(i)]);
 }
 
 // Variant with the A operand in LDS (built once per block, read per MFMA; ≈37 KB next to the
@@ -1565,9 +1567,9 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab3_mixed(const float* __restr
                                                       const uint32_t* __restrict__ str_a,
                                                       const uint16_t* __restrict__ outT, int npp, int np,
                                                       const float* __restrict__ vpk, int nmt) {
-    extern __shared__ __attribute__((aligned(16))) double srow_m3[];  // [Nb] then A operands
+    extern __shared__ __attribute__((aligned(16))) double srow_m3[];  // [ab_row_slots(Nb)] then A operands
     double* srow = srow_m3;
-    bf8* Ash = reinterpret_cast<bf8*>(srow + ((Nb + 1) & ~int64_t(1)));  // [nmt][KS][2][64]
+    bf8* Ash = reinterpret_cast<bf8*>(srow + ab_row_slots(Nb));  // [nmt][KS][2][64]
     __shared__ uint32_t ent[KS * 32];
     __shared__ __attribute__((aligned(16))) float vdg[12 * 16];
     constexpr int NTH = 64 * WM * WC, NW = WM * WC;
@@ -1577,7 +1579,7 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab3_mixed(const float* __restr
     const int wm = wave % WM, wc = wave / WM;
     const int g = lane >> 4, cl = lane & 15;
     for (int i = tid; i < KS * 32; i += NTH) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
-    for (int64_t i = tid; i < Nb; i += NTH) srow[i] = 0.0;
+    for (int i = tid; i < int(ab_row_slots(Nb)); i += NTH) srow[i] = 0.0;
     const uint32_t occ = str_a[Ja];
     for (int r = tid; r < nmt * 16; r += NTH) {  // diagonal excitations: sum_{q in Ja} (qq|r)
         float d = 0.f;
@@ -1633,7 +1635,6 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab3_mixed(const float* __restr
         d = *reinterpret_cast<const float2*>(Crow + Ibc);
     };
     auto compute = [&](const float2 (&x)[KS][8], const uint4 (&t)[TPW], float2 cd, int64_t c0) {
-        const bool ok = c0 + 2 * cl < Nb;
         bf8 bh0[KS], bl0[KS], bh1[KS], bl1[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
@@ -1670,10 +1671,10 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab3_mixed(const float* __restr
             for (int p = 0; p < 2; ++p)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const uint32_t tt = (tw[p * 2 + v / 2] >> (16 * (v & 1))) & 0xFFFFu;
-                    if (!ok || (tt & 0x7FFFu) == kInv16) continue;
+                    const uint32_t w = tw[p * 2 + v / 2];
                     const float a = (p ? a1[v] : a0[v]) + vd4[v] * (p ? cd.y : cd.x);
-                    atomicAdd(&srow[tt & 0x7FFFu], double((tt >> 15) ? -a : a));
+                    atomicAdd(&srow[ab_target(w, v & 1)],
+                              double(__uint_as_float(__float_as_uint(a) ^ ab_sign(w, v & 1))));
                 }
         }
     };
@@ -1691,16 +1692,13 @@ __global__ __launch_bounds__(64 * WM * WC) void k_ab3_mixed(const float* __restr
     }
     __syncthreads();
     float* Srow = S + Ja * Nb;
-    for (int64_t i = tid; i < Nb; i += NTH) Srow[i] = float(double(Srow[i]) + srow[i]);
+    for (int i = tid; i < int(Nb); i += NTH) Srow[i] = float(double(Srow[i]) + srow[ab_slot(i)]);
 }
 
 // FP64: 16x16x4 MFMA, KS k-steps of 4 single excitations. The A operand rows are loaded in the
 // permuted order m -> rs = 4 (m % 4) + m / 4 inside each tile so that the accumulator element v of
 // lane (g = lane / 16) is row rs = 4 g + v, the layout of the 16-bit target table.
-// SPLIT (nmt = 4 (TPW - 1) + 1): the last row tile is shared by the four row-tile waves, each
-// taking a quarter of its k-steps and scattering its partial product, so every wave runs
-// 2 (TPW - 1) + KS / 4 MFMA chains' worth of k-steps instead of one wave running TPW full tiles.
-template <int KS, int TPW, bool SPLIT>
+template <int KS>
 __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C, double* __restrict__ S, int64_t Na,
                                                     int64_t Nb, const uint32_t* __restrict__ into_a, int ns,
                                                     const uint32_t* __restrict__ str_a,
@@ -1710,7 +1708,7 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
                                                     const double* const* __restrict__ C_t = nullptr,
                                                     double* const* __restrict__ S_t = nullptr,
                                                     const double* const* __restrict__ V_t = nullptr) {
-    extern __shared__ __attribute__((aligned(16))) double srow64[];  // [Nb]
+    extern __shared__ __attribute__((aligned(16))) double srow64[];  // [ab_row_slots(Nb)]
     if (act) {
         if (!act[blockIdx.y]) return;
         C = C_t[blockIdx.y];
@@ -1719,14 +1717,14 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
     }
     __shared__ uint32_t ent[KS * 4];
     __shared__ double vdg[12 * 16];
-    constexpr int WM = 4, WC = 2, NTH = 64 * WM * WC;
+    constexpr int TPW = 3, WM = 4, WC = 2, NTH = 64 * WM * WC;
     const int64_t Ja = xcd_remap(blockIdx.x, Na);
     if (Ja >= Na) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wc = wave / WM;
     const int g = lane >> 4, cl = lane & 15;
     for (int i = tid; i < KS * 4; i += NTH) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
-    for (int64_t i = tid; i < Nb; i += NTH) srow64[i] = 0.0;
+    for (int i = tid; i < int(ab_row_slots(Nb)); i += NTH) srow64[i] = 0.0;
     const uint32_t occ = str_a[Ja];
     for (int r = tid; r < nmt * 16; r += NTH) {  // diagonal excitations: sum_{q in Ja} (qq|r)
         double d = 0.0;
@@ -1738,28 +1736,10 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
         vdg[r] = d;
     }
     __syncthreads();
-    constexpr int TF = SPLIT ? TPW - 1 : TPW;  // full row tiles per wave
-    constexpr int KQ = KS / 4;                  // k-steps of the shared tile per wave
-    static_assert(!SPLIT || KS % 4 == 0, "shared tile needs KS divisible by 4");
-    double va[TF][KS];
-    double vd[TF][4];
-    double vs[SPLIT ? KQ : 1], vds[4];
-    const int mts = WM * (TPW - 1);  // the shared tile
-    if constexpr (SPLIT) {
-        const int rs = mts * 16 + 4 * (cl % 4) + cl / 4;
+    double va[TPW][KS];
+    double vd[TPW][4];
 #pragma unroll
-        for (int q = 0; q < KQ; ++q) {
-            const int e = (wm * KQ + q) * 4 + g;
-            const uint32_t en = ent[e];
-            const bool use = mts < nmt && rs < np && e < ns && en != kInvalid;
-            const double t = vpk[use ? size_t((en >> 21) & 0x3FFu) * np + rs : 0];
-            vs[q] = use ? ((en >> 31) ? -t : t) : 0.0;
-        }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) vds[v] = wm == 0 && mts < nmt ? vdg[mts * 16 + 4 * g + v] : 0.0;  // once
-    }
-#pragma unroll
-    for (int j = 0; j < TF; ++j) {
+    for (int j = 0; j < TPW; ++j) {
         const int mtile = wm + WM * j;
         const int rs = mtile * 16 + 4 * (cl % 4) + cl / 4;  // permuted A row
 #pragma unroll
@@ -1782,7 +1762,7 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
         const int64_t Ibc = Ib < Nb ? Ib : 0;  // columns past the end: computed, never scattered
 #pragma unroll
         for (int j = 0; j < TPW; ++j) {
-            const int mtile = SPLIT && j == TPW - 1 ? mts : wm + WM * j;  // the table row c0 / 32 exists
+            const int mtile = wm + WM * j;  // the table row c0 / 32 exists
             const int mtc = mtile < nmt ? mtile : 0;  // for all lanes; tiles past nmt are skipped below
             tg[j] = *reinterpret_cast<const uint4*>(outT + (((c0 >> 5) * ntile + mtc) * 64 + lane) * 8);
         }
@@ -1797,10 +1777,9 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
     int64_t c0 = int64_t(wc) * 32;
     if (c0 < Nb) load(c0, xv, tg, cd);
     for (; c0 < Nb; c0 += 32 * WC) {
-        const bool ok = c0 + 2 * cl < Nb;
         d4 acc0[TPW], acc1[TPW];
 #pragma unroll
-        for (int j = 0; j < TF; ++j) {
+        for (int j = 0; j < TPW; ++j) {
             acc0[j] = d4{0.0, 0.0, 0.0, 0.0};
             acc1[j] = d4{0.0, 0.0, 0.0, 0.0};
             if (wm + WM * j >= nmt) continue;  // wave-uniform
@@ -1808,23 +1787,6 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
             for (int ks = 0; ks < KS; ++ks) {
                 acc0[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[j][ks], xv[ks].x, acc0[j], 0, 0, 0);
                 acc1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[j][ks], xv[ks].y, acc1[j], 0, 0, 0);
-            }
-        }
-        if constexpr (SPLIT) {
-            acc0[TPW - 1] = d4{0.0, 0.0, 0.0, 0.0};
-            acc1[TPW - 1] = d4{0.0, 0.0, 0.0, 0.0};
-            if (mts < nmt) {  // this wave's quarter of the shared tile's k-steps (compile-time indices)
-#pragma unroll
-                for (int w = 0; w < WM; ++w)
-                    if (wm == w) {
-#pragma unroll
-                        for (int q = 0; q < KQ; ++q) {
-                            acc0[TPW - 1] =
-                                __builtin_amdgcn_mfma_f64_16x16x4f64(vs[q], xv[w * KQ + q].x, acc0[TPW - 1], 0, 0, 0);
-                            acc1[TPW - 1] =
-                                __builtin_amdgcn_mfma_f64_16x16x4f64(vs[q], xv[w * KQ + q].y, acc1[TPW - 1], 0, 0, 0);
-                        }
-                    }
             }
         }
         uint4 tgc[TPW];
@@ -1838,23 +1800,20 @@ __global__ __launch_bounds__(512, 2) void k_ab2_f64(const double* __restrict__ C
             for (int p = 0; p < 2; ++p)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const uint32_t tt = (tw[p * 2 + v / 2] >> (16 * (v & 1))) & 0xFFFFu;
-                    if (!ok || (tt & 0x7FFFu) == kInv16) continue;
+                    const uint32_t w = tw[p * 2 + v / 2];
                     const double a = (p ? a1[v] : a0[v]) + vdj[v] * (p ? cdc.y : cdc.x);
-                    atomicAdd(&srow64[tt & 0x7FFFu], (tt >> 15) ? -a : a);
+                    atomicAdd(&srow64[ab_target(w, v & 1)], ab_sign(w, v & 1) ? -a : a);
                 }
         };
 #pragma unroll
-        for (int j = 0; j < TF; ++j) {
+        for (int j = 0; j < TPW; ++j) {
             if (wm + WM * j >= nmt) continue;  // wave-uniform
             scatter(tgc[j], acc0[j], acc1[j], vd[j]);
         }
-        if constexpr (SPLIT)
-            if (mts < nmt) scatter(tgc[TPW - 1], acc0[TPW - 1], acc1[TPW - 1], vds);
     }
     __syncthreads();
     double* Srow = S + Ja * Nb;
-    for (int64_t i = tid; i < Nb; i += NTH) Srow[i] += srow64[i];
+    for (int i = tid; i < int(Nb); i += NTH) Srow[i] += srow64[ab_slot(i)];
 }
 
 __global__ void k_clique_diag(const uint32_t* __restrict__ str, int64_t nstr, int n, int d,
@@ -2157,11 +2116,11 @@ static void ab_mixed_launch(const float* C, float* S, const SpinTables& a, const
     HIPCHK(hipGetLastError());
 }
 
-template <int KS, int TPW, bool SPLIT>
+template <int KS>
 static void ab2_f64_launch(const double* C, double* S, const SpinTables& a, const SpinTables& b,
                            const DevInts& ints, hipStream_t st, bool half) {
-    const size_t sh = size_t(b.nstr) * sizeof(double);
-    auto kern = k_ab2_f64<KS, TPW, SPLIT>;
+    const size_t sh = size_t(ab_row_slots(b.nstr)) * sizeof(double);
+    auto kern = k_ab2_f64<KS>;
     HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
     kern<<<xcd_grid(a.nstr), 512, sh, st>>>(C, S, a.nstr, b.nstr, a.into.p, a.ns, a.str.p, b.outT.p, b.npp, b.np,
                                             (half ? ints.vpk_h.p : ints.vpk.p), (b.np + 15) / 16, nullptr, nullptr, nullptr, nullptr);
@@ -2171,7 +2130,7 @@ template <int KS, int TPW, int WM, int WC>
 static void ab3_mixed_launch(const float* C, float* S, const SpinTables& a, const SpinTables& b,
                              const DevInts& ints, hipStream_t st, bool half) {
     const int nmt = (b.np + 15) / 16;
-    const size_t sh3 = size_t((b.nstr + 1) & ~int64_t(1)) * sizeof(double) + size_t(nmt) * KS * 2 * 64 * 16;
+    const size_t sh3 = size_t(ab_row_slots(b.nstr)) * sizeof(double) + size_t(nmt) * KS * 2 * 64 * 16;
     if (nmt > WM * TPW || sh3 + KS * 32 * 4 + 12 * 16 * 4 > 160 * 1024)
         throw Error(-1, "alpha-beta kernel: LDS A-operand layout does not fit this shape");
     auto kern3 = k_ab3_mixed<KS, TPW, WM, WC>;
@@ -2184,7 +2143,7 @@ static void ab3_mixed_launch(const float* C, float* S, const SpinTables& a, cons
 template <int KS, int TPW, int WM, int WC>
 static void ab2_mixed_launch(const float* C, float* S, const SpinTables& a, const SpinTables& b,
                              const DevInts& ints, hipStream_t st, bool half) {
-    const size_t sh = size_t(b.nstr) * sizeof(double);
+    const size_t sh = size_t(ab_row_slots(b.nstr)) * sizeof(double);
     auto kern = k_ab2_mixed<KS, TPW, WM, WC>;
     HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
     kern<<<xcd_grid(a.nstr), 64 * WM * WC, sh, st>>>(C, S, a.nstr, b.nstr, a.into.p, a.ns, a.str.p, b.outT.p, b.npp, b.np,
@@ -2195,25 +2154,26 @@ static void ab2_mixed_launch(const float* C, float* S, const SpinTables& a, cons
 // register-resident kernels: 16-bit targets, LDS row, E <= 96, <= 12 row tiles
 static bool ab2_ok(const SpinTables& a, const SpinTables& b, size_t w) {
     return b.outT.p != nullptr && b.nstr % 2 == 0 && a.ns <= 96 && (b.np + 15) / 16 <= 12 &&
-           size_t(b.nstr) * w <= 150 * 1024;
+           size_t(ab_row_slots(b.nstr)) * w <= 150 * 1024;
 }
+
+// The FP64 kernel without LDS staging takes what fci_ab64.hip's cannot hold beside a row of 15.8 to
+// 19.2 thousand strings (18 orbitals with 6 or 12 beta electrons): 9 to 12 row tiles
+static bool ab2_f64_ok(const SpinTables& a, const SpinTables& b) {
+    return ab2_ok(a, b, sizeof(double)) && (b.np + 15) / 16 > 8;
+}
+static int ab2_f64_ks(const SpinTables& a) { return std::max(1, (a.ns + 15) / 16) * 4; }
 
 static void launch_ab(const double* C, double* S, const SpinTables& a, const SpinTables& b,
                       const DevInts& ints, hipStream_t st, bool half) {
-    if (ab2_ok(a, b, sizeof(double))) {
-        const int ks = std::max(1, (a.ns + 15) / 16) * 4;  // k-steps of 4, in buckets of 16 excitations
-        const int tpw = ((b.np + 15) / 16 + 3) / 4;
-        // nmt = 4 (tpw - 1) + 1: the last row tile shared by the four row-tile waves
-        const bool split = tpw > 1 && (b.np + 15) / 16 == 4 * (tpw - 1) + 1;
-#define F64CASE(K, T)                                                                      \
-    if (ks == K && tpw == T)                                                                \
-        return split ? ab2_f64_launch<K, T, (T > 1)>(C, S, a, b, ints, st, half)                  \
-                     : ab2_f64_launch<K, T, false>(C, S, a, b, ints, st, half);
-#define F64ROW(K) F64CASE(K, 1) F64CASE(K, 2) F64CASE(K, 3)
-        F64ROW(4) F64ROW(8) F64ROW(12) F64ROW(16) F64ROW(20) F64ROW(24)
-#undef F64ROW
+    if (ab5_f64_ok(a, b)) return ab5_f64(C, S, a, b, half ? ints.vpk_h.p : ints.vpk.p, st);
+    if (ab2_f64_ok(a, b)) {
+        switch (ab2_f64_ks(a)) {
+#define F64CASE(K) \
+    case K: return ab2_f64_launch<K>(C, S, a, b, ints, st, half);
+            F64CASE(4) F64CASE(8) F64CASE(12) F64CASE(16) F64CASE(20) F64CASE(24)
 #undef F64CASE
-        throw Error(-1, "alpha-beta kernel: no instance for this shape");
+        }
     }
     int ks = std::max(1, (a.ns + 3) / 4);
     if ((b.np + 15) / 16 > 4 * AB_MTW) throw Error(-1, "too many orbitals for the alpha-beta kernel");
@@ -2258,7 +2218,7 @@ static void launch_ab(const float* C, float* S, const SpinTables& a, const SpinT
             MXCASE(3, 1) MXCASE(3, 2)
 #undef MXCASE
         }
-        const size_t sh3 = size_t((b.nstr + 1) & ~int64_t(1)) * 8 + size_t(nmt) * ks * 2 * 64 * 16 + 1024 + 768;
+        const size_t sh3 = size_t(ab_row_slots(b.nstr)) * 8 + size_t(nmt) * ks * 2 * 64 * 16 + 1024 + 768;
         if (layout == 1 && sh3 <= 160 * 1024) {
 #define MXCASE(K, T) \
     if (ks == K && nmt == T) return ab3_mixed_launch<K, T, 1, 8>(C, S, a, b, ints, st, half);
@@ -2299,10 +2259,7 @@ bool batch_sigma_supported(const SpinTables& a, const SpinTables& b, std::string
     if (a.M > 64 || b.M > 64 || (a.M + 3) / 4 > 16 || (b.M + 3) / 4 > 16)
         return no("batched sigma: same-spin cliques too large");
     if (a.nstr % 2 || b.nstr % 2) return no("batched sigma needs even string counts");
-    if (!ab2_ok(a, b, sizeof(double))) return no("batched sigma: alpha-beta shape not supported");
-    const int ks = std::max(1, (a.ns + 15) / 16) * 4;
-    const int tpw = ((b.np + 15) / 16 + 3) / 4;
-    if (ks > 24 || tpw > 3) return no("batched sigma: alpha-beta shape not supported");
+    if (!ab5_f64_ok(a, b) && !ab2_f64_ok(a, b)) return no("batched sigma: alpha-beta shape not supported");
     return true;
 }
 
@@ -2349,31 +2306,29 @@ static void batch_clique_f64(const SpinTables& sp, int gd, int64_t L, const void
     HIPCHK(hipGetLastError());
 }
 
-template <int KS, int TPW, bool SPLIT>
+template <int KS>
 static void batch_ab2_f64(const SpinTables& a, const SpinTables& b, const BatchSigmaTabs& t, hipStream_t st) {
-    const size_t sh = size_t(b.nstr) * sizeof(double);  // attribute set by batch_sigma_prepare
-    auto kern = k_ab2_f64<KS, TPW, SPLIT>;
+    const size_t sh = size_t(ab_row_slots(b.nstr)) * sizeof(double);  // attribute set by batch_sigma_prepare
+    auto kern = k_ab2_f64<KS>;
     kern<<<dim3(xcd_grid(a.nstr), unsigned(t.nitem)), 512, sh, st>>>(
         nullptr, nullptr, a.nstr, b.nstr, a.into.p, a.ns, a.str.p, b.outT.p, b.npp, b.np, nullptr, (b.np + 15) / 16,
         t.act, t.c, t.s, t.vpk);
     HIPCHK(hipGetLastError());
 }
 
-template <int KS, int TPW, bool SPLIT> static void batch_ab2_attr(const SpinTables& b) {
-    HIPCHK(hipFuncSetAttribute((const void*)k_ab2_f64<KS, TPW, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(size_t(b.nstr) * sizeof(double))));
+template <int KS> static void batch_ab2_attr(const SpinTables& b) {
+    HIPCHK(hipFuncSetAttribute((const void*)k_ab2_f64<KS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               int(size_t(ab_row_slots(b.nstr)) * sizeof(double))));
 }
 
 void batch_sigma_prepare(const SpinTables& a, const SpinTables& b) {
-    const int ks = std::max(1, (a.ns + 15) / 16) * 4;
-    const int tpw = ((b.np + 15) / 16 + 3) / 4;
-    const bool split = tpw > 1 && (b.np + 15) / 16 == 4 * (tpw - 1) + 1;
-#define F64CASE(K, T) \
-    if (ks == K && tpw == T) return split ? batch_ab2_attr<K, T, (T > 1)>(b) : batch_ab2_attr<K, T, false>(b);
-#define F64ROW(K) F64CASE(K, 1) F64CASE(K, 2) F64CASE(K, 3)
-    F64ROW(4) F64ROW(8) F64ROW(12) F64ROW(16) F64ROW(20) F64ROW(24)
-#undef F64ROW
+    if (ab5_f64_ok(a, b)) return ab5_f64_prepare(a, b);
+    switch (ab2_f64_ks(a)) {
+#define F64CASE(K) \
+    case K: return batch_ab2_attr<K>(b);
+        F64CASE(4) F64CASE(8) F64CASE(12) F64CASE(16) F64CASE(20) F64CASE(24)
 #undef F64CASE
+    }
     throw Error(-1, "batched alpha-beta kernel: no instance for this shape");
 }
 
@@ -2417,16 +2372,13 @@ void batch_sigma_f64_ms0(const SpinTables& a, const SpinTables& b, int gd_a, int
 }
 
 static void batch_ab_f64(const SpinTables& a, const SpinTables& b, const BatchSigmaTabs& t, hipStream_t st) {
-    const int ks = std::max(1, (a.ns + 15) / 16) * 4;
-    const int tpw = ((b.np + 15) / 16 + 3) / 4;
-    const bool split = tpw > 1 && (b.np + 15) / 16 == 4 * (tpw - 1) + 1;
-#define F64CASE(K, T)                                                                              \
-    if (ks == K && tpw == T)                                                                        \
-        return split ? batch_ab2_f64<K, T, (T > 1)>(a, b, t, st) : batch_ab2_f64<K, T, false>(a, b, t, st);
-#define F64ROW(K) F64CASE(K, 1) F64CASE(K, 2) F64CASE(K, 3)
-    F64ROW(4) F64ROW(8) F64ROW(12) F64ROW(16) F64ROW(20) F64ROW(24)
-#undef F64ROW
+    if (ab5_f64_ok(a, b)) return ab5_f64_batch(a, b, t, st);
+    switch (ab2_f64_ks(a)) {
+#define F64CASE(K) \
+    case K: return batch_ab2_f64<K>(a, b, t, st);
+        F64CASE(4) F64CASE(8) F64CASE(12) F64CASE(16) F64CASE(20) F64CASE(24)
 #undef F64CASE
+    }
     throw Error(-1, "batched alpha-beta kernel: no instance for this shape");
 }
 

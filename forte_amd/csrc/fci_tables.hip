@@ -180,7 +180,7 @@ static inline unsigned nblk(int64_t n, int bs) { return unsigned((n + bs - 1) / 
 // 16 tile + 4 g + v (v = 0..3):
 //   element (((it * ntile + tile) * 64 + 16 g + c) * 2 + p) * 4 + v,  string 32 it + 2c + p,
 // so the 8 targets a lane needs for one tile are one 16-byte word and a wave's 64 words are
-// contiguous. Strings beyond nstr and pairs beyond np hold 0x7FFF (none).
+// contiguous. Strings beyond nstr and pairs beyond np hold an unused slot too.
 __global__ void k_out_t16(const uint32_t* __restrict__ out, int64_t nstr, int np, int npp, uint16_t* __restrict__ o16) {
     const int ntile = npp / 16;
     const int64_t nrow = (nstr + 31) / 32 * 32;
@@ -194,10 +194,13 @@ __global__ void k_out_t16(const uint32_t* __restrict__ out, int64_t nstr, int np
     const int64_t it = q / ntile;
     const int64_t I = it * 32 + 2 * (lane % 16) + pp;
     const int P = tile * 16 + 4 * (lane / 16) + v;
-    uint16_t val = 0x7FFFu;
+    // none: of the 64 unused slots one that no other lane of a wave takes, whether its lanes hold 16
+    // consecutive strings or every other one of 32
+    const int col = int(I & 31);
+    uint16_t val = uint16_t((nstr + 31) / 32 * 32 + 16 * (lane / 16) + ((col >> 1) & 7) + 8 * ((col ^ (col >> 4)) & 1));
     if (P < np && I < nstr) {
         const uint32_t t = out[int64_t(P) * nstr + I];
-        if (t != kInvalid) val = uint16_t((t & kAddrMask) | ((t >> 31) << 15));
+        if (t != kInvalid) val = uint16_t(ab_slot(int(t & kAddrMask)) | ((t >> 31) << 15));
     }
     o16[x] = val;
 }
@@ -217,7 +220,7 @@ void build_spin_tables(SpinTables& t, int n, int k, const uint32_t* B, hipStream
     t.np = n * (n + 1) / 2;
     t.out.alloc(size_t(t.nstr) * t.np);
     k_out<<<nblk(t.nstr * t.np, 256), 256, 0, st>>>(t.str.p, t.out.p, t.nstr, n, t.np, B);
-    if (t.nstr <= 32767) {
+    if (ab_row_slots(t.nstr) <= 32768) {
         t.npp = (t.np + 15) / 16 * 16;
         const int64_t nrow = (t.nstr + 31) / 32 * 32;
         t.outT.alloc(size_t(nrow) * t.npp);

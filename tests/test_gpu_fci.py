@@ -79,6 +79,24 @@ def test_sigma_fp64(oracle, n, na, nb):
     assert np.abs(got - ref).max() < 1e-12 * scale
 
 
+# The FP64 alpha-beta kernel at the edges of its 16-column chunks and k-steps: odd string counts, one
+# string, fewer strings than a chunk (15), exactly one (16), one more than a whole number of them, 3 to 0
+# free excitation slots, and every row-tile count of 1 to 9 with and without padding pairs.
+AB64_CASES = [(5, 2, 3), (5, 4, 5), (7, 3, 4), (7, 4, 1), (8, 3, 4), (8, 1, 7), (9, 4, 3), (11, 5, 3), (11, 2, 9),
+              (13, 4, 2), (13, 2, 4), (13, 1, 12), (15, 2, 2), (15, 13, 1), (15, 3, 14), (16, 1, 1), (16, 2, 15),
+              (16, 15, 2)]
+
+
+@pytest.mark.parametrize("n,na,nb", AB64_CASES)
+def test_sigma_fp64_chunk_edges(oracle, n, na, nb):
+    say("sigma fp64 edges", n, na, nb)
+    p = seeded_problem(n, na, nb, 27 + n, e_core=-0.4)
+    g, o = gpu_solver(p), cpu_oracle(oracle, p)
+    C = np.random.default_rng(n * 10 + nb).standard_normal(o.ndet)
+    ref = o.sigma(C)
+    assert np.abs(g.sigma(C) - ref).max() < 1e-12 * max(1.0, np.abs(ref).max())
+
+
 @pytest.mark.parametrize("n,na,nb", [(6, 3, 3), (8, 4, 4), (10, 5, 5), (12, 6, 6), (9, 3, 5), (14, 3, 3), (16, 2, 2),
                                      (16, 3, 3), (17, 2, 2), (18, 3, 3),
                                      # same-spin cliques of 36, 45 and 55 members (the alpha side,
