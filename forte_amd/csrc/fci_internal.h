@@ -91,7 +91,7 @@ struct SpinTables {
     // tile layout [ceil(nstr/32)][npp/16][64 lanes][2][4] (npp = np rounded up to 16): the 8 targets of
     // lane (g, c) for strings 32 it + 2c + p and pairs 16 tile + 4 g + v are one 16-byte word, and each
     // string's 4 are one 8-byte word; string J has slot ab_slot(J), and an excitation that does not
-    // exist has one of the 64 unused slots behind the row. Built only when the slots fit in 15 bits.
+    // exist has one of the 128 unused slots behind the row. Built only when the slots fit in 15 bits.
     int npp = 0;
     DBuf<uint16_t> outT;
     // pair cliques for the same-spin operator: hole strings K with k-d electrons (d = 2, or 1
@@ -109,11 +109,11 @@ struct SpinTables {
 // The row of sigma that an alpha-beta kernel accumulates in LDS: within 32 strings the even ones come
 // first, so that both 16 consecutive strings and every other one of 32 fall into 16 different banks
 // (FP64 LDS atomics of a wave, 4 runs of 16 strings: 8.3 cycles, against 16.2 for every other string of
-// a row in plain order). Behind the strings, 64 slots that absorb what does not exist: without a
+// a row in plain order). Behind the strings, 128 slots that absorb what does not exist: without a
 // divergent branch a scattered value takes 5 vector instructions instead of 11, and inactive lanes save
 // an atomic nothing (8.1 cycles with half of them).
 __host__ __device__ inline int ab_slot(int J) { return (J & ~31) | ((J & 1) << 4) | ((J >> 1) & 15); }
-__host__ __device__ inline int64_t ab_row_slots(int64_t nstr) { return (nstr + 31) / 32 * 32 + 64; }
+__host__ __device__ inline int64_t ab_row_slots(int64_t nstr) { return (nstr + 31) / 32 * 32 + 128; }
 
 void build_spin_tables(SpinTables& t, int n, int k, const uint32_t* d_binom, hipStream_t st);
 // point-group classes of the strings: irrep (XOR of the occupied orbitals' irreps, orbsym in
@@ -253,6 +253,9 @@ bool ab5_f64_ok(const SpinTables& a, const SpinTables& b);
 void ab5_f64(const double* C, double* S, const SpinTables& a, const SpinTables& b, const double* vpk, hipStream_t st);
 void ab5_f64_batch(const SpinTables& a, const SpinTables& b, const BatchSigmaTabs& t, hipStream_t st);
 void ab5_f64_prepare(const SpinTables& a, const SpinTables& b);
+// the mixed-precision one (fci_ab32.hip)
+bool ab5_mixed_ok(const SpinTables& b);
+void ab5_mixed(const float* C, float* S, const SpinTables& a, const SpinTables& b, const float* vpk, hipStream_t st);
 // sets the kernel attributes batch_sigma_f64 needs (call before capturing it in a graph)
 void batch_sigma_prepare(const SpinTables& a, const SpinTables& b);
 void batch_sigma_f64(const SpinTables& a, const SpinTables& b, int gd_a, int gd_b, const BatchSigmaTabs& t,

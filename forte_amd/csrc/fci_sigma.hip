@@ -2190,48 +2190,25 @@ static void launch_ab(const double* C, double* S, const SpinTables& a, const Spi
 }
 static void launch_ab(const float* C, float* S, const SpinTables& a, const SpinTables& b,
                       const DevInts& ints, hipStream_t st, bool half) {
+    if (ab5_mixed_ok(b)) return ab5_mixed(C, S, a, b, half ? ints.vpk32_h.p : ints.vpk32.p, st);
     if (ab2_ok(a, b, sizeof(double))) {
+        // From 9 row tiles (16 orbitals) on. 9 and 10: 8 waves each on its own 32 columns and all row
+        // tiles, the A operand in LDS, the next tile's loads in flight (15.0 ms at CAS(16,16), against
+        // 15.5 ms for ab5_mixed, whose A operands take the registers of the second wave a SIMD).
+        // Otherwise 8 waves as 2 row-tile groups x 4 column groups with A in registers.
         const int ks = std::max(1, (a.ns + 31) / 32);
         const int nmt = (b.np + 15) / 16;
-        // Default for 3..10 row tiles: 8 waves each on its own 32 columns and all row tiles, the A
-        // operand in LDS, the next tile's loads in flight (k_ab3_mixed<K, T, 1, 8>: 16.5 ms at
-        // CAS(16,16)); otherwise 8 waves as 2 row-tile groups x 4 column groups with A in
-        // registers (k_ab2_mixed<K, T, 2, 4>: 19.7 ms there, each X tile loaded by two waves).
-        // FCI_AB_LAYOUT=8 forces the latter, 12 and 3 select 4 x 3 and 3 x 4 groups.
-        static const int layout = [] {
-            const char* e = std::getenv("FCI_AB_LAYOUT");
-            return e ? std::atoi(e) : 1;
-        }();
-        if (layout == 3 && (nmt + 2) / 3 * ks <= 6) {
-            const int tpw = (nmt + 2) / 3;
-#define MXCASE(K, T) \
-    if (ks == K && tpw == T) return ab2_mixed_launch<K, T, 3, 4>(C, S, a, b, ints, st, half);
-            MXCASE(1, 1) MXCASE(1, 2) MXCASE(1, 3) MXCASE(1, 4) MXCASE(2, 1) MXCASE(2, 2) MXCASE(2, 3)
-            MXCASE(3, 1) MXCASE(3, 2)
-#undef MXCASE
-        }
-        if (layout == 12 && (nmt + 3) / 4 * ks <= 6) {
-            const int tpw = (nmt + 3) / 4;
-#define MXCASE(K, T) \
-    if (ks == K && tpw == T) return ab2_mixed_launch<K, T, 4, 3>(C, S, a, b, ints, st, half);
-            MXCASE(1, 1) MXCASE(1, 2) MXCASE(1, 3) MXCASE(2, 1) MXCASE(2, 2) MXCASE(2, 3)
-            MXCASE(3, 1) MXCASE(3, 2)
-#undef MXCASE
-        }
         const size_t sh3 = size_t(ab_row_slots(b.nstr)) * 8 + size_t(nmt) * ks * 2 * 64 * 16 + 1024 + 768;
-        if (layout == 1 && sh3 <= 160 * 1024) {
+        if (sh3 <= 160 * 1024) {
 #define MXCASE(K, T) \
     if (ks == K && nmt == T) return ab3_mixed_launch<K, T, 1, 8>(C, S, a, b, ints, st, half);
-            MXCASE(1, 3) MXCASE(1, 4) MXCASE(1, 5) MXCASE(1, 6) MXCASE(1, 7) MXCASE(1, 8) MXCASE(1, 9) MXCASE(1, 10)
-            MXCASE(2, 3) MXCASE(2, 4) MXCASE(2, 5) MXCASE(2, 6) MXCASE(2, 7) MXCASE(2, 8) MXCASE(2, 9) MXCASE(2, 10)
+            MXCASE(1, 9) MXCASE(1, 10) MXCASE(2, 9) MXCASE(2, 10)
 #undef MXCASE
         }
         const int tpw = (nmt + 1) / 2;
 #define MXCASE(K, T) \
     if (ks == K && tpw == T) return ab2_mixed_launch<K, T, 2, 4>(C, S, a, b, ints, st, half);
-#define MXROW(K) MXCASE(K, 1) MXCASE(K, 2) MXCASE(K, 3) MXCASE(K, 4) MXCASE(K, 5) MXCASE(K, 6)
-        MXROW(1) MXROW(2) MXROW(3)
-#undef MXROW
+        MXCASE(1, 5) MXCASE(1, 6) MXCASE(2, 5) MXCASE(2, 6) MXCASE(3, 5) MXCASE(3, 6)
 #undef MXCASE
         throw Error(-1, "alpha-beta kernel: no instance for this shape");
     }

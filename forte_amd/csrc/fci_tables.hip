@@ -180,29 +180,45 @@ static inline unsigned nblk(int64_t n, int bs) { return unsigned((n + bs - 1) / 
 // 16 tile + 4 g + v (v = 0..3):
 //   element (((it * ntile + tile) * 64 + 16 g + c) * 2 + p) * 4 + v,  string 32 it + 2c + p,
 // so the 8 targets a lane needs for one tile are one 16-byte word and a wave's 64 words are
-// contiguous. Strings beyond nstr and pairs beyond np hold an unused slot too.
+// contiguous. Strings beyond nstr and pairs beyond np have no target either. One thread per half of an
+// instruction of the mixed kernels (32 lanes: 2 pairs x 16 every-other strings): the lanes without a
+// target take unused slots in the banks that the others leave free, so that they cost nothing.
 __global__ void k_out_t16(const uint32_t* __restrict__ out, int64_t nstr, int np, int npp, uint16_t* __restrict__ o16) {
     const int ntile = npp / 16;
-    const int64_t nrow = (nstr + 31) / 32 * 32;
+    const int64_t nit = (nstr + 31) / 32;
     const int64_t x = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (x >= nrow * npp) return;
-    const int v = int(x % 4);
-    const int pp = int((x / 4) % 2);
-    const int lane = int((x / 8) % 64);
-    const int64_t q = x / 512;  // it * ntile + tile
+    if (x >= nit * ntile * 16) return;
+    const int v = int(x % 4), pp = int((x / 4) % 2), h = int((x / 8) % 2);
+    const int64_t q = x / 16;  // it * ntile + tile
     const int tile = int(q % ntile);
     const int64_t it = q / ntile;
-    const int64_t I = it * 32 + 2 * (lane % 16) + pp;
-    const int P = tile * 16 + 4 * (lane / 16) + v;
-    // none: of the 64 unused slots one that no other lane of a wave takes, whether its lanes hold 16
-    // consecutive strings or every other one of 32
-    const int col = int(I & 31);
-    uint16_t val = uint16_t((nstr + 31) / 32 * 32 + 16 * (lane / 16) + ((col >> 1) & 7) + 8 * ((col ^ (col >> 4)) & 1));
-    if (P < np && I < nstr) {
-        const uint32_t t = out[int64_t(P) * nstr + I];
-        if (t != kInvalid) val = uint16_t(ab_slot(int(t & kAddrMask)) | ((t >> 31) << 15));
+    uint16_t* o = o16 + (q * 64 + 32 * h) * 8 + pp * 4 + v;
+    uint32_t val[32], banks = 0;  // banks: of the targets that exist
+#pragma unroll
+    for (int l = 0; l < 32; ++l) {
+        const int64_t I = it * 32 + 2 * (l % 16) + pp;
+        const int P = tile * 16 + 4 * (2 * h + l / 16) + v;
+        val[l] = P < np && I < nstr ? out[int64_t(P) * nstr + I] : kInvalid;
     }
-    o16[x] = val;
+#pragma unroll
+    for (int l = 0; l < 32; ++l)
+        if (val[l] != kInvalid) {
+            const uint32_t s = uint32_t(ab_slot(int(val[l] & kAddrMask)));
+            banks |= 1u << (s & 31u);
+            val[l] = s | (val[l] >> 31) << 15;
+        } else {
+            val[l] = 0x10000u;
+        }
+    const uint32_t none = uint32_t((nstr + 31) / 32 * 32) + 64 * pp + 32 * h;
+#pragma unroll
+    for (int l = 0; l < 32; ++l) {
+        if (val[l] == 0x10000u) {  // as many banks are free as there are lanes without a target, or more
+            const int f = __ffs(~banks) - 1;
+            banks |= 1u << f;
+            val[l] = none + uint32_t(f);
+        }
+        o[l * 8] = uint16_t(val[l]);
+    }
 }
 
 void build_spin_tables(SpinTables& t, int n, int k, const uint32_t* B, hipStream_t st) {
@@ -224,7 +240,7 @@ void build_spin_tables(SpinTables& t, int n, int k, const uint32_t* B, hipStream
         t.npp = (t.np + 15) / 16 * 16;
         const int64_t nrow = (t.nstr + 31) / 32 * 32;
         t.outT.alloc(size_t(nrow) * t.npp);
-        k_out_t16<<<nblk(nrow * t.npp, 256), 256, 0, st>>>(t.out.p, t.nstr, t.np, t.npp, t.outT.p);
+        k_out_t16<<<nblk(nrow * t.npp / 32, 64), 64, 0, st>>>(t.out.p, t.nstr, t.np, t.npp, t.outT.p);
     }
     t.d = k >= 2 ? 2 : (k == 1 ? 1 : 0);
     if (t.d > 0) {

@@ -127,6 +127,28 @@ def test_sigma_mixed(oracle, n, na, nb):
     assert err < (3e-6 if n >= 16 else 6e-7)
 
 
+# The mixed alpha-beta kernel at the edges of its 32-column chunks, for odd rows (the last column is read
+# with the one before it), one and two k-steps, one and two row waves; bounds as above, the few-electron
+# 15-orbital shapes like the 16-orbital ones.
+@pytest.mark.parametrize("n,na,nb", [(4, 1, 3), (5, 3, 2), (7, 3, 4), (7, 4, 1), (8, 1, 3), (9, 4, 2), (11, 2, 4), (12, 3, 1),
+                                     (13, 2, 4), (13, 4, 1), (13, 4, 12), (14, 4, 13), (15, 2, 2), (15, 3, 1), (15, 1, 14)])
+def test_sigma_mixed_chunk_edges(oracle, n, na, nb):
+    import forte_amd
+    say("sigma mixed edges", n, na, nb)
+    p = seeded_problem(n, na, nb, 37 + n)
+    g, o = gpu_solver(p), cpu_oracle(oracle, p)
+    C = np.random.default_rng(n + 100 * nb).standard_normal(o.ndet)
+    C /= np.linalg.norm(C)
+    ref = o.sigma(C)
+    c32 = forte_amd.DeviceArray(o.ndet, "float32")
+    s32 = forte_amd.DeviceArray(o.ndet, "float32")
+    c32.upload(C.astype(np.float32))
+    g.sigma_arrays(c32, s32)
+    err = np.linalg.norm(s32.download().astype(np.float64) - ref) / np.linalg.norm(ref)
+    say("  relative error", err)
+    assert err < (3e-6 if n >= 15 else 6e-7)
+
+
 def test_sigma_device_fp64_matches_host(oracle):
     import forte_amd
     p = seeded_problem(8, 4, 4, 5)
