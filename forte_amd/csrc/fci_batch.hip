@@ -762,7 +762,7 @@ struct BatchClass {
     SpinTables sa, sb;
     DBuf<uint32_t> binom;
     int gd[2] = {0, 0};
-    DBuf<double> g2a, g2b, vpk, vpkh, hd, b, sg, r, tmp, tms, part, scratch;
+    DBuf<double> g2a, g2b, hsa, hsb, vpk, vpkh, hd, b, sg, r, tmp, tms, part, scratch;
     // Ms = 0 spin-flip symmetry (C^T = eta C): the Davidson-Liu vectors are packed coordinates
     // (nd of them) of full vectors of ndf = N^2 determinants, and sigma has no beta same-spin term
     int eta = 0;
@@ -772,7 +772,8 @@ struct BatchClass {
     DBuf<int64_t> pvoff, pidx;
     DBuf<double> pval;
     // sigma tables
-    DBuf<const double*> c_tab, g2a_tab, g2b_tab, vpk_tab, vpkh_tab;
+    DBuf<const double*> c_tab, g2a_tab, g2b_tab, ha_tab, hb_tab, vpk_tab, vpkh_tab;
+    bool dense = false;  // same-spin operators as dense matrices (hsa, hsb)
     DBuf<double*> s_tab, ct_tab, yt_tab, e_tab;
     hipStream_t stream = nullptr;
     int* done_host = nullptr;
@@ -849,6 +850,10 @@ struct BatchClass {
             t.e = e_tab.p;
             t.g2a = g2a_tab.p + i0;
             t.g2b = g2b_tab.p + i0;
+            if (dense) {
+                t.ha = ha_tab.p + i0;
+                t.hb = eta ? nullptr : hb_tab.p + i0;
+            }
             if (eta) {
                 t.vpk = vpkh_tab.p + i0;
                 batch_sigma_f64_ms0(sa, sb, gd[0], eta, t, stream);
@@ -1074,6 +1079,29 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
             }
             C.g2a.alloc(g2a_h.size()); C.g2a.upload(g2a_h.data(), g2a_h.size());
             C.g2b.alloc(g2b_h.size()); C.g2b.upload(g2b_h.data(), g2b_h.size());
+            // small spaces: the dense same-spin operators of every problem (the symmetric form has no
+            // beta term), unless they would take more memory than a few classes' vectors
+            const size_t ha2 = size_t(C.sa.nstr) * C.sa.nstr, hb2 = C.eta ? 0 : size_t(C.sb.nstr) * C.sb.nstr;
+            C.dense = dense_same_use(C.sa, C.sb, sizeof(double)) && size_t(P) * (ha2 + hb2) * 8 <= (size_t(16) << 30);
+            if (C.dense) {
+                C.hsa.alloc(size_t(P) * ha2);
+                if (hb2) C.hsb.alloc(size_t(P) * hb2);
+                for (int spin = 0; spin < (hb2 ? 2 : 1); ++spin) {
+                    const size_t h2 = spin ? hb2 : ha2, gg = size_t(C.gd[spin]) * C.gd[spin];
+                    std::vector<const double*> gp(P);
+                    std::vector<double*> hp(P);
+                    for (int q = 0; q < P; ++q) {
+                        gp[q] = (spin ? C.g2b.p : C.g2a.p) + size_t(q) * gg;
+                        hp[q] = (spin ? C.hsb.p : C.hsa.p) + size_t(q) * h2;
+                    }
+                    DBuf<const double*> dg(P);
+                    DBuf<double*> dh(P);
+                    dg.upload(gp.data(), P);
+                    dh.upload(hp.data(), P);
+                    dense_same_batch(spin ? C.sb : C.sa, dg.p, C.gd[spin], dh.p, P, C.stream);
+                    HIPCHK(hipStreamSynchronize(C.stream));
+                }
+            }
             C.vpk.alloc(vpk_h.size()); C.vpk.upload(vpk_h.data(), vpk_h.size());
             if (C.eta) {  // halved packed integrals (exact) for the symmetric sigma
                 for (double& x : vpk_h) x *= 0.5;
@@ -1097,7 +1125,7 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
             const int nitem = P * C.NSL;
             std::vector<int> sbs = {nitem};
             size_t oyt = 0, oe = 0;
-            const size_t scr = batch_sigma_scratch_elems(C.sa, C.sb, &oyt, &oe);
+            const size_t scr = batch_sigma_scratch_elems(C.sa, C.sb, C.dense, &oyt, &oe);
             if (nitem > 16 && scr * 8 * size_t(nitem) > (size_t(8) << 30)) sbs.push_back(16);
             for (int64_t x : chls)
                 for (int y : sbs) C.var.push_back({x, y});
@@ -1128,11 +1156,13 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
             C.pidx.alloc(pidx.size()); C.pidx.upload(pidx.data(), pidx.size());
             C.pval.alloc(pval.size()); C.pval.upload(pval.data(), pval.size());
             // sigma tables: per item integrals, per slot scratch
-            std::vector<const double*> ga(nitem), gb2(nitem), vp(nitem), vph(nitem);
+            std::vector<const double*> ga(nitem), gb2(nitem), vp(nitem), vph(nitem), ha(nitem), hb(nitem);
             for (int it = 0; it < nitem; ++it) {
                 const int q = it / C.NSL;
                 ga[it] = C.g2a.p + size_t(q) * C.gd[0] * C.gd[0];
                 gb2[it] = C.g2b.p + size_t(q) * C.gd[1] * C.gd[1];
+                ha[it] = C.dense ? C.hsa.p + size_t(q) * ha2 : nullptr;
+                hb[it] = C.dense && hb2 ? C.hsb.p + size_t(q) * hb2 : nullptr;
                 vp[it] = C.vpk.p + size_t(q) * size_t(n * (n + 1) / 2) * size_t(n * (n + 1) / 2);
                 vph[it] = C.eta ? C.vpkh.p + size_t(q) * size_t(n * (n + 1) / 2) * size_t(n * (n + 1) / 2) : nullptr;
             }
@@ -1145,6 +1175,8 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
             C.c_tab.alloc(nitem); C.s_tab.alloc(nitem);
             C.g2a_tab.alloc(nitem); C.g2a_tab.upload(ga.data(), nitem);
             C.g2b_tab.alloc(nitem); C.g2b_tab.upload(gb2.data(), nitem);
+            C.ha_tab.alloc(nitem); C.ha_tab.upload(ha.data(), nitem);
+            C.hb_tab.alloc(nitem); C.hb_tab.upload(hb.data(), nitem);
             C.vpk_tab.alloc(nitem); C.vpk_tab.upload(vp.data(), nitem);
             C.vpkh_tab.alloc(nitem); C.vpkh_tab.upload(vph.data(), nitem);
             C.ct_tab.alloc(slots); C.ct_tab.upload(ct.data(), slots);

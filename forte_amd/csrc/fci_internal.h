@@ -164,6 +164,11 @@ struct DevInts {
     DBuf<float> g2f_off[2];
     DBuf<float> gdiag[2];
     int gdim[2] = {0, 0};
+    // the same-spin operators of small spaces as dense matrices (fci_dense.hip); empty where the cliques
+    // are used. hs[1] stays empty when both spins have the same one.
+    DBuf<double> hs[2];
+    bool dense = false;
+    const double* same(int spin) const { return hs[spin && hs[1].p ? 1 : 0].p; }
 };
 
 // Host copy of the integrals in Forte's layout (the guess and packing work on the host).
@@ -243,10 +248,26 @@ struct BatchSigmaTabs {
     const double* const* g2a = nullptr;
     const double* const* g2b = nullptr;
     const double* const* vpk = nullptr;
+    const double* const* ha = nullptr;  // dense same-spin operators (else the cliques, with e, g2a, g2b)
+    const double* const* hb = nullptr;
 };
 bool batch_sigma_supported(const SpinTables& a, const SpinTables& b, std::string* why);
-// elements of scratch per item; *off_yt and *off_e: offsets of Y^T and E inside it (C^T at 0)
-size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, size_t* off_yt, size_t* off_e);
+// elements of scratch per item; *off_yt and *off_e: offsets of Y^T and E inside it (C^T at 0); dense: no E
+size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, bool dense, size_t* off_yt, size_t* off_e);
+// ---- dense same-spin operators of small spaces (fci_dense.hip) -----------------------------------
+// whether sigma with w-byte elements uses them; the operator of one spin (nstr x nstr) from its cliques,
+// for one problem and for several of one shape; S (+)= scale C + Ha C + C Hb (null: no such term), for one
+// vector and for the items of a batch
+bool dense_same_use(const SpinTables& a, const SpinTables& b, size_t w);
+void dense_same_device(const SpinTables& sp, const double* d_g, int gdim, double* d_h, hipStream_t st);
+void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, double* const* h_t, int nprob,
+                      hipStream_t st);
+template <class T>
+void dense_same_apply(const T* C, T* S, int64_t Na, int64_t Nb, const double* Ha, const double* Hb, T scale, bool add,
+                      hipStream_t st);
+void dense_same_apply_batch(int64_t Na, int64_t Nb, int nitem, const void* const* act, const double* const* C_t,
+                            double* const* S_t, const double* const* Ha_t, const double* const* Hb_t, hipStream_t st);
+
 // the FP64 alpha-beta term with the gathered rows staged in LDS (fci_ab64.hip): whether it takes these
 // tables, sigma += H_ab C with the packed integrals vpk, the batched form and its kernel attributes
 bool ab5_f64_ok(const SpinTables& a, const SpinTables& b);

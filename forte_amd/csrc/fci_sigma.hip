@@ -2242,14 +2242,14 @@ bool batch_sigma_supported(const SpinTables& a, const SpinTables& b, std::string
 
 static int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, size_t* off_yt, size_t* off_e) {
+size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, bool dense, size_t* off_yt, size_t* off_e) {
     const size_t nd = size_t(a.nstr) * size_t(b.nstr);
     const size_t v = (nd + 31) & ~size_t(31);  // 256-byte aligned in FP64
     const size_t ea = size_t(a.nK) * a.M * size_t(round_up(b.nstr, CQ3_CW));
     const size_t eb = size_t(b.nK) * b.M * size_t(round_up(a.nstr, CQ3_CW));
     if (off_yt) *off_yt = v;
     if (off_e) *off_e = 2 * v;
-    return 2 * v + std::max(ea, eb);
+    return 2 * v + (dense ? 0 : std::max(ea, eb));
 }
 
 static void batch_clique_f64(const SpinTables& sp, int gd, int64_t L, const void* const* act,
@@ -2315,6 +2315,10 @@ void batch_sigma_f64(const SpinTables& a, const SpinTables& b, int gd_a, int gd_
                      hipStream_t st) {
     const int64_t Na = a.nstr, Nb = b.nstr;
     const unsigned ni = unsigned(t.nitem);
+    if (t.ha) {
+        dense_same_apply_batch(Na, Nb, t.nitem, t.act, t.c, t.s, t.ha, t.hb, st);
+        return batch_ab_f64(a, b, t, st);
+    }
     // beta same-spin on C^T: C -> C^T, cliques -> Y^T, sigma = (Y^T)^T
     k_transpose64<double><<<dim3(nblk(Nb, 64), nblk(Na, 64), ni), 256, 0, st>>>(nullptr, nullptr, Na, Nb, nullptr,
                                                                                0.0, t.act, t.c, t.ct, nullptr);
@@ -2340,7 +2344,10 @@ void batch_sigma_f64_ms0(const SpinTables& a, const SpinTables& b, int gd_a, int
     BatchSigmaTabs u = t;
     u.c = t.ct;
     u.s = t.yt;
-    batch_clique_f64(a, gd_a, N, u.act, u.c, u.e, u.g2a, u.s, false, u.nitem, st);
+    if (t.ha)
+        dense_same_apply_batch(N, N, t.nitem, t.act, t.ct, t.yt, t.ha, nullptr, st);
+    else
+        batch_clique_f64(a, gd_a, N, u.act, u.c, u.e, u.g2a, u.s, false, u.nitem, st);
     batch_ab_f64(a, b, u, st);
     // packed coordinates of sigma = S + eta S^T
     k_ms0_pack<double, double><<<dim3(tg, tg, ni), 256, 0, st>>>(nullptr, nullptr, N, eta == 1 ? 0 : 1, eta,
@@ -2399,9 +2406,14 @@ void SigmaEngine::apply_t(const T* C, T* S, hipStream_t st, unsigned char* ext, 
         eext = ext + off;
         eext_bytes = ext_bytes - off;
     }
+    const bool dense = ints_->dense && dense_same_use(a, b, sizeof(T));
     if (timing_) HIPCHK(hipEventRecord(w_->ev[0], st));
-    // beta same-spin on C^T, then sigma = (Y^T) + e_core C   (H0, fci_vector_hamiltonian.cc:84-91)
-    if (b.d > 0) {
+    // small spaces: e_core C and both same-spin terms in one dense product (timed as the beta one);
+    // otherwise beta same-spin on C^T, then sigma = (Y^T) + e_core C   (H0, fci_vector_hamiltonian.cc:84-91)
+    if (dense) {
+        dense_same_apply<T>(C, S, Na, Nb, a.d > 0 ? ints_->same(0) : nullptr, b.d > 0 ? ints_->same(1) : nullptr, ecore,
+                            false, st);
+    } else if (b.d > 0) {
         if (!ext) {
             DBuf<T>& Ct = scratch<T>(*w_, 0);
             DBuf<T>& Yt = scratch<T>(*w_, 1);
@@ -2417,7 +2429,7 @@ void SigmaEngine::apply_t(const T* C, T* S, hipStream_t st, unsigned char* ext, 
         k_scale_copy<T><<<nblk(nd, 256), 256, 0, st>>>(C, S, nd, ecore);
     }
     if (timing_) HIPCHK(hipEventRecord(w_->ev[1], st));
-    if (a.d > 0) launch_clique<T>(C, S, Nb, a, *ints_, 0, true, *w_, st, eext, eext_bytes);
+    if (a.d > 0 && !dense) launch_clique<T>(C, S, Nb, a, *ints_, 0, true, *w_, st, eext, eext_bytes);
     if (timing_) HIPCHK(hipEventRecord(w_->ev[2], st));
     if (a.k > 0 && b.k > 0) launch_ab(C, S, a, b, *ints_, st, false);
     if (timing_) {
@@ -2443,13 +2455,18 @@ void SigmaEngine::apply_sym_t(const T* C, T* S, int eta, hipStream_t st, bool in
     if (a.nstr != b.nstr || a.k != b.k) throw Error(-1, "sigma: the spin-flip form needs equal alpha and beta strings");
     if (eta != 1 && eta != -1) throw Error(-1, "sigma: eta must be +1 or -1");
     const int64_t N = a.nstr, nd = N * N;
+    const bool dense = ints_->dense && dense_same_use(a, b, sizeof(T));
     if (timing_) HIPCHK(hipEventRecord(w_->ev[0], st));
-    if (init) {
+    if (init && !dense) {
         k_scale_copy<T><<<nblk(nd, 256), 256, 0, st>>>(C, S, nd, T(0.5 * ints_->e_core));
         HIPCHK(hipGetLastError());
     }
     if (timing_) HIPCHK(hipEventRecord(w_->ev[1], st));
-    if (a.d > 0) launch_clique<T>(C, S, N, a, *ints_, 0, true, *w_, st, nullptr, 0);
+    if (dense)
+        dense_same_apply<T>(C, S, N, N, a.d > 0 ? ints_->same(0) : nullptr, nullptr,
+                            init ? T(0.5 * ints_->e_core) : T(0), !init, st);
+    else if (a.d > 0)
+        launch_clique<T>(C, S, N, a, *ints_, 0, true, *w_, st, nullptr, 0);
     if (timing_) HIPCHK(hipEventRecord(w_->ev[2], st));
     if (a.k > 0) launch_ab(C, S, a, b, *ints_, st, true);
     if (finish) sym_add_device<T>(S, N, eta, false, st);

@@ -417,6 +417,21 @@ class Solver {
                 HIPCHK(hipStreamSynchronize(0));
             }
         }
+        di_.dense = dense_same_use(sa_, sb_, sizeof(double));
+        if (di_.dense) {
+            const bool shared = na_ == nb_ && pk.g2[0] == pk.g2[1];
+            for (int spin = 0; spin < 2; ++spin) {
+                const SpinTables& sp = spin ? sb_ : sa_;
+                if (shared && spin) {
+                    di_.hs[1].release();
+                    continue;
+                }
+                const size_t need = sp.d > 0 ? size_t(sp.nstr) * sp.nstr : 0;
+                if (di_.hs[spin].n != need) di_.hs[spin].alloc(need);
+                if (need) dense_same_device(sp, di_.g2[spin].p, di_.gdim[spin], di_.hs[spin].p, 0);
+            }
+            HIPCHK(hipStreamSynchronize(0));
+        }
         have_ints_ = true;
     }
 

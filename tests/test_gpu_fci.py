@@ -149,6 +149,27 @@ def test_sigma_mixed_chunk_edges(oracle, n, na, nb):
     assert err < (3e-6 if n >= 15 else 6e-7)
 
 
+# The dense same-spin product: ragged tiles of 32 and 64 and ragged k chunks in both products, 64 x 64
+# tiles (924 x 792), one of the two terms missing, one-electron operators.
+@pytest.mark.parametrize("n,na,nb", [(6, 0, 3), (6, 3, 0), (7, 3, 1), (9, 2, 2), (12, 2, 1), (12, 6, 1), (12, 1, 6),
+                                     (11, 5, 4), (12, 6, 0), (12, 6, 5)])
+def test_sigma_dense_same_spin(oracle, n, na, nb):
+    import forte_amd
+    say("dense same spin", n, na, nb)
+    p = seeded_problem(n, na, nb, 47 + n, e_core=0.9)
+    g, o = gpu_solver(p), cpu_oracle(oracle, p)
+    C = np.random.default_rng(3 * n + nb).standard_normal(o.ndet)
+    C /= np.linalg.norm(C)
+    ref = o.sigma(C)
+    assert np.abs(g.sigma(C) - ref).max() < 1e-12 * max(1.0, np.abs(ref).max())
+    c32 = forte_amd.DeviceArray(o.ndet, "float32")
+    s32 = forte_amd.DeviceArray(o.ndet, "float32")
+    c32.upload(C.astype(np.float32))
+    g.sigma_arrays(c32, s32)
+    err = np.linalg.norm(s32.download().astype(np.float64) - ref) / np.linalg.norm(ref)
+    assert err < 6e-7  # as test_sigma_mixed
+
+
 def test_sigma_device_fp64_matches_host(oracle):
     import forte_amd
     p = seeded_problem(8, 4, 4, 5)
