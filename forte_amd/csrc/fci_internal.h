@@ -390,6 +390,11 @@ void rdm1_device(const SpinTables& a, const SpinTables& b, const double* L, cons
                  double* g1a, double* g1b, hipStream_t st);
 void rdm2_same_device(const SpinTables& a, const SpinTables& b, const double* L, const double* R,
                       double* g2aa, double* g2bb, hipStream_t st);
+// the same on FP64 MFMA for up to 16 orbitals (fci_rdm2.hip), adding to cleared outputs
+bool rdm2_ab5_ok(const SpinTables& a, const SpinTables& b);
+void rdm2_ab5(const SpinTables& a, const SpinTables& b, const double* L, const double* R, double* g2ab, hipStream_t st);
+bool rdm2_clique5_ok(const SpinTables& sp, int64_t ncol);
+void rdm2_clique5(const SpinTables& sp, const double* L, const double* R, int64_t ncol, double* acc, int gdim, hipStream_t st);
 void rdm2_ab_device(const SpinTables& a, const SpinTables& b, const double* L, const double* R,
                     double* g2ab, hipStream_t st);
 double spin2_device(const SpinTables& a, const SpinTables& b, const double* L, const double* R,

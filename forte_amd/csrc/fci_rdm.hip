@@ -5,6 +5,8 @@
 // g2ss[p][q][r][s] = <L| a+p a+q a_s a_r |R>            same spin, through the pair cliques:
 //                   sum_K <L|a+p a+q|K><K|a_s a_r|R>, a dense M x M product per hole string K
 // g2ab[p][r][q][s] = <L| E^a_pq E^b_rs |R>              per alpha row, singles x beta excitations
+// (the 2-RDM kernels here take what fci_rdm2.hip does not: 17 orbitals and up, cliques of more than 64
+// members, single columns)
 // <S^2> = -sum_rs <E^a_sr E^b_rs> + (na-nb)^2/4 + (na+nb)/2
 #include "fci_internal.h"
 
@@ -631,10 +633,15 @@ void rdm1_device(const SpinTables& a, const SpinTables& b, const double* L, cons
     if (a.ns + 1 > RD_MAXE || b.ns + 1 > RD_MAXE) throw Error(-1, "rdm1: too many excitations per string");
     if (a.k > 0) k_rdm1_rows<<<unsigned(Na), RD_BS, 0, st>>>(L, R, Na, Nb, a.into.p, a.ns, a.str.p, n, g1a);
     if (b.k > 0) {
-        DBuf<double> Lt(size_t(Na) * Nb), Rt(size_t(Na) * Nb);
+        DBuf<double> Lt(size_t(Na) * Nb), Rt;
         transpose_device<double>(L, Lt.p, Na, Nb, st);
-        transpose_device<double>(R, Rt.p, Na, Nb, st);
-        k_rdm1_rows<<<unsigned(Nb), RD_BS, 0, st>>>(Lt.p, Rt.p, Nb, Na, b.into.p, b.ns, b.str.p, n, g1b);
+        const double* rt = Lt.p;
+        if (R != L) {
+            Rt.alloc(size_t(Na) * Nb);
+            transpose_device<double>(R, Rt.p, Na, Nb, st);
+            rt = Rt.p;
+        }
+        k_rdm1_rows<<<unsigned(Nb), RD_BS, 0, st>>>(Lt.p, rt, Nb, Na, b.into.p, b.ns, b.str.p, n, g1b);
         HIPCHK(hipStreamSynchronize(st));
     }
     HIPCHK(hipGetLastError());
@@ -647,18 +654,28 @@ void rdm2_same_device(const SpinTables& a, const SpinTables& b, const double* L,
     const int npair = a.n * (a.n - 1) / 2;
     HIPCHK(hipMemsetAsync(acc_a, 0, size_t(npair) * npair * sizeof(double), st));
     HIPCHK(hipMemsetAsync(acc_b, 0, size_t(npair) * npair * sizeof(double), st));
-    if (a.d == 2) {
+    if (a.d == 2 && rdm2_clique5_ok(a, Nb)) {
+        rdm2_clique5(a, L, R, Nb, acc_a, npair, st);
+    } else if (a.d == 2) {
         const int nta = (a.M + RC_MAXM - 1) / RC_MAXM;
         k_rdm2_clique<<<dim3(unsigned(a.nK), unsigned(nta * nta)), RD_BS, 0, st>>>(L, R, Nb, a.clq.p, a.M, acc_a, npair,
                                                                                   nta);
     }
     if (b.d == 2) {
         const int ntb = (b.M + RC_MAXM - 1) / RC_MAXM;
-        DBuf<double> Lt(size_t(Na) * Nb), Rt(size_t(Na) * Nb);
+        DBuf<double> Lt(size_t(Na) * Nb), Rt;
         transpose_device<double>(L, Lt.p, Na, Nb, st);
-        transpose_device<double>(R, Rt.p, Na, Nb, st);
-        k_rdm2_clique<<<dim3(unsigned(b.nK), unsigned(ntb * ntb)), RD_BS, 0, st>>>(Lt.p, Rt.p, Na, b.clq.p, b.M, acc_b,
-                                                                                   npair, ntb);
+        const double* rt = Lt.p;
+        if (R != L) {
+            Rt.alloc(size_t(Na) * Nb);
+            transpose_device<double>(R, Rt.p, Na, Nb, st);
+            rt = Rt.p;
+        }
+        if (rdm2_clique5_ok(b, Na))
+            rdm2_clique5(b, Lt.p, rt, Na, acc_b, npair, st);
+        else
+            k_rdm2_clique<<<dim3(unsigned(b.nK), unsigned(ntb * ntb)), RD_BS, 0, st>>>(Lt.p, rt, Na, b.clq.p, b.M, acc_b,
+                                                                                       npair, ntb);
         HIPCHK(hipStreamSynchronize(st));
     }
     HIPCHK(hipGetLastError());
@@ -669,6 +686,7 @@ void rdm2_ab_device(const SpinTables& a, const SpinTables& b, const double* L, c
     const int n = a.n;
     HIPCHK(hipMemsetAsync(g2ab, 0, size_t(n) * n * n * n * sizeof(double), st));
     if (a.k == 0 || b.k == 0) return;
+    if (rdm2_ab5_ok(a, b)) return rdm2_ab5(a, b, L, R, g2ab, st);
     if (a.ns + a.k > RD_MAXE) throw Error(-1, "rdm2ab: too many excitations per string");
     // MFMA kernel when every output tile of a row has a wave slot and the chunks fit in LDS
     const int ET = (a.ns + a.k + 15) / 16, ZT = (2 * b.np + 15) / 16;

@@ -1572,18 +1572,44 @@ int fci_rdms(fci_solver* s, int rl, int rr, int level, double* g1a, double* g1b,
         const size_t n2 = size_t(n) * n, n4 = n2 * n2;
         const double* L = S.evec_device(rl);
         const double* R = S.evec_device(rr);
-        fci::DBuf<double> d1a(n2), d1b(n2);
-        fci::rdm1_device(S.sa_, S.sb_, L, R, d1a.p, d1b.p, 0);
-        HIPCHK(hipStreamSynchronize(0));
-        if (g1a) d1a.download(g1a, n2);
-        if (g1b) d1b.download(g1b, n2);
+        // with the alpha-beta 2-RDM at hand the 1-RDMs are its partial traces, sum_r <E^alpha_pq E^beta_rr> =
+        // nb <E^alpha_pq>; otherwise from the vectors
+        const bool traced = level >= 2 && S.na_ > 0 && S.nb_ > 0;
+        if (!traced) {
+            fci::DBuf<double> d1a(n2), d1b(n2);
+            fci::rdm1_device(S.sa_, S.sb_, L, R, d1a.p, d1b.p, 0);
+            HIPCHK(hipStreamSynchronize(0));
+            if (g1a) d1a.download(g1a, n2);
+            if (g1b) d1b.download(g1b, n2);
+        }
         if (level >= 2) {
             const int np = n * (n - 1) / 2;
             fci::DBuf<double> aa(size_t(np > 0 ? np : 1) * (np > 0 ? np : 1)), bb(aa.n), ab(n4);
             fci::rdm2_same_device(S.sa_, S.sb_, L, R, aa.p, bb.p, 0);
             fci::rdm2_ab_device(S.sa_, S.sb_, L, R, ab.p, 0);
             HIPCHK(hipStreamSynchronize(0));
-            if (g2ab) ab.download(g2ab, n4);
+            if (traced && (g1a || g1b || g2ab)) {
+                std::vector<double> own;
+                double* g = g2ab;
+                if (!g) {
+                    own.resize(n4);
+                    g = own.data();
+                }
+                ab.download(g, n4);
+                auto at = [&](int p, int r, int q, int t) { return g[((size_t(p) * n + r) * n + q) * n + t]; };
+                for (int p = 0; p < n; ++p)
+                    for (int q = 0; q < n; ++q) {
+                        double ta = 0.0, tb = 0.0;
+                        for (int r = 0; r < n; ++r) {
+                            ta += at(p, r, q, r);
+                            tb += at(r, p, r, q);
+                        }
+                        if (g1a) g1a[size_t(p) * n + q] = ta / S.nb_;
+                        if (g1b) g1b[size_t(p) * n + q] = tb / S.na_;
+                    }
+            } else if (g2ab) {
+                ab.download(g2ab, n4);
+            }
             // expand the pair matrices with the reference's fill (fci_vector_rdm.cc:240-285): the
             // element of the larger pair index is copied to its transpose
             for (int spin = 0; spin < 2; ++spin) {

@@ -240,6 +240,25 @@ def test_rdms_vs_oracle(oracle):
     assert abs(e - g.energies()[0]) < 1e-9
 
 
+@pytest.mark.parametrize("n,na,nb", [(5, 2, 1), (5, 1, 2), (7, 3, 2), (9, 4, 5), (10, 5, 3), (11, 2, 2), (12, 6, 2),
+                                     (13, 2, 6), (14, 7, 1), (16, 8, 1), (16, 1, 8)])
+def test_rdms_tile_edges(oracle, n, na, nb):
+    """1- and 2-RDMs over every count of excitation, pair and clique tiles, odd and even rows, one and two vectors."""
+    say("rdms tiles", n, na, nb)
+    p = seeded_problem(n, na, nb, 43)
+    g, o = gpu_solver(p, 2, abs(na - nb) + 1), cpu_oracle(oracle, p)
+    g.set_e_convergence(1e-6)
+    g.set_r_convergence(1e-4)
+    g.set_maxiter(300)
+    g.compute_energy()
+    # sums over at most 2e5 products of two unit vectors' entries: 1e-12 is some 10^3 eps of the largest element
+    for (l, r) in [(0, 0), (0, 1)]:
+        rd = g.rdms([(l, r)], 2)[0]
+        ref = o.rdms(g.evec(l), g.evec(r))
+        for a, b in zip([rd.g1a(), rd.g1b(), rd.g2aa(), rd.g2ab(), rd.g2bb()], ref):
+            assert np.abs(a - b).max() < 1e-12, (l, r)
+
+
 def test_rdms_against_oracle_eigenvector(oracle):
     """Root 0 RDMs of the GPU solve agree with the oracle's own solve (sign-invariant)."""
     p = seeded_problem(8, 4, 4, 1)
