@@ -115,3 +115,21 @@ def test_dl_errors():
         forte_amd.DavidsonLiuSolver(4, 1, 2, 2)
     with pytest.raises(RuntimeError):
         forte_amd.DavidsonLiuSolver(0, 1)
+
+
+@pytest.mark.parametrize("size", [3, 300])
+def test_dl_guess_entries(size):
+    """Guesses of many entries, over the edge of a block, with indices given twice (the later value stands): exact
+    eigenvectors as guesses are converged at once, to rounding (some 1e-13 of a spectrum of at most 30)."""
+    import forte_amd
+    M = synthetic(size)
+    w, V = np.linalg.eigh(M)
+    s = forte_amd.DavidsonLiuSolver(size, 2)
+    s.add_h_diag(np.diag(M).copy())
+    s.add_guesses([[(i, 7.0) for i in range(0, size, 2)] + [(i, V[i, k]) for i in range(size)] for k in range(2)])
+    s.add_test_sigma_builder(M)
+    s.set_maxiter(3)
+    s.solve()
+    assert np.abs(np.asarray(s.eigenvalues()[:2]) - w[:2]).max() < 1e-11
+    for k in range(2):
+        assert abs(abs(np.dot(s.eigenvector(k), V[:, k])) - 1.0) < 1e-11
