@@ -72,6 +72,19 @@ def test_transforms_and_diagonal_vs_oracle(oracle, n, na, nb, twoS, orbsym, irre
     assert np.abs(s.hdiag_csf() - np.diag(T @ H @ T.T)).max() < 1e-11
 
 
+@pytest.mark.parametrize("n,na,nb,twoS", [(3, 2, 1, 1), (9, 5, 4, 1), (10, 5, 5, 0)])
+def test_hdiag_many_open_shells(oracle, n, na, nb, twoS):
+    """CSF diagonals with rows of a few and of many determinants (one a thread, one a wave), one configuration
+    and thousands; sums of weights adding up to 1 of diagonals of order 10: 1e-11 is 10^3 eps of that."""
+    from oracle.spin_adapt import SpinAdapter
+    say(f"csf diagonal n={n} na={na} nb={nb} 2S={twoS}")
+    p = seeded_problem(n, na, nb, 13)
+    s = solver(p, 1, twoS + 1, None, 0)
+    ref = SpinAdapter(n, na, nb, twoS, None, 0)
+    o = oracle.Oracle(n, na, nb, p["h"], p["h"], p["aa"], p["ab"], p["aa"], p["e_core"])
+    assert np.abs(s.hdiag_csf() - ref.hdiag(o.hdiag())).max() < 1e-11
+
+
 @pytest.mark.parametrize("n,na,nb,twoS", [(18, 2, 2, 0), (17, 3, 1, 2), (18, 3, 2, 1)])
 def test_transforms_beyond_16_orbitals_vs_oracle(n, na, nb, twoS):
     """Above 16 orbitals the string ranks are summed electron by electron (the byte tables cover
