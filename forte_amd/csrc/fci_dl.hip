@@ -76,42 +76,14 @@ template <int N> struct Coefs {
     }
 };
 
-// out_part[blk][i] = sum over this block's elements of x[e] * Y_i[e]  (i < m)
-template <class TX, class TY>  // FP64 or FP32 vectors (FP32 sigma rows of the mixed phase), FP64 sums
-__global__ __launch_bounds__(DL_BS) void k_dots(const TX* __restrict__ x, const TY* __restrict__ Y,
-                                                int m, int64_t n, double* __restrict__ part) {
-    __shared__ double red[DL_MAXM][DL_BS / 64];
-    double acc[DL_MAXM];
-#pragma unroll
-    for (int i = 0; i < DL_MAXM; ++i) acc[i] = 0.0;
-    for (int64_t e = int64_t(blockIdx.x) * DL_BS + threadIdx.x; e < n; e += int64_t(gridDim.x) * DL_BS) {
-        double xv = double(x[e]);
-#pragma unroll
-        for (int i = 0; i < DL_MAXM; ++i)
-            if (i < m) acc[i] += xv * double(Y[size_t(i) * n + e]);
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < DL_MAXM; ++i) {
-        if (i >= m) break;
-        double v = acc[i];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-        if (lane == 0) red[i][wave] = v;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < m; i += DL_BS) {
-        double s = 0.0;
-        for (int w = 0; w < DL_BS / 64; ++w) s += red[i][w];
-        part[size_t(blockIdx.x) * m + i] = s;
-    }
-}
-
-// part[blk][i] for the vectors i of chunk blockIdx.y (8 per chunk), double2 loads (x and every
-// Y_i 16-byte aligned: n even)
+// part[blk][i] = this block's share of x . Y_i (i < m) for the vectors i of chunk blockIdx.y (8 per chunk). FP64 or
+// FP32 vectors (FP32 sigma rows of the mixed phase), FP64 sums. Pairs of elements a load, at the alignment of one
+// element: rows of odd length take the same path, their last entry by itself (on average over a solve with 382,239
+// CSFs 8.7 us; single elements with 64 sums held took 38).
 constexpr int DOT_MC = 8;
 template <class T> struct Vec2;
-template <> struct Vec2<double> { using type = double2; };
-template <> struct Vec2<float> { using type = float2; };
+template <> struct Vec2<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct Vec2<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
 template <class TX, class TY>
 __global__ __launch_bounds__(DL_BS) void k_dots8(const TX* __restrict__ x, const TY* __restrict__ Y, int m,
                                                  int64_t n, double* __restrict__ part) {
@@ -133,6 +105,12 @@ __global__ __launch_bounds__(DL_BS) void k_dots8(const TX* __restrict__ x, const
                 const Y2 y = reinterpret_cast<const Y2*>(Y + size_t(i0 + i) * n)[e];
                 acc[i] += double(xv.x) * double(y.x) + double(xv.y) * double(y.y);
             }
+    }
+    if (n % 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+        const double xv = double(x[n - 1]);
+#pragma unroll
+        for (int i = 0; i < DOT_MC; ++i)
+            if (i < mc) acc[i] += xv * double(Y[size_t(i0 + i) * n + n - 1]);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -574,17 +552,8 @@ void DavidsonLiu::dots_t(const TX* x, const TY* Y, int m, double* out) {
     if (m <= 0) return;
     double* part = part_.p;
     double* res = part_.p + size_t(DL_NBLK) * DL_MAXM;
-    int nb;
-    // two-element loads need every vector aligned to two elements: even lengths only
-    if (m <= DL_MAXM && size_ % 2 == 0 && reinterpret_cast<uintptr_t>(x) % (2 * sizeof(TX)) == 0 &&
-        reinterpret_cast<uintptr_t>(Y) % (2 * sizeof(TY)) == 0) {
-        nb = int(std::min<int64_t>(DL_NBLK, (size_ / 2 + DL_BS - 1) / DL_BS));
-        nb = std::max(nb, 1);
-        k_dots8<TX, TY><<<dim3(nb, (m + DOT_MC - 1) / DOT_MC), DL_BS>>>(x, Y, m, size_, part);
-    } else {
-        nb = int(std::min<int64_t>(DL_NBLK, (size_ + DL_BS - 1) / DL_BS));
-        k_dots<TX, TY><<<nb, DL_BS>>>(x, Y, m, size_, part);
-    }
+    const int nb = int(std::max<int64_t>(1, std::min<int64_t>(DL_NBLK, (size_ / 2 + DL_BS - 1) / DL_BS)));
+    k_dots8<TX, TY><<<dim3(nb, (m + DOT_MC - 1) / DOT_MC), DL_BS>>>(x, Y, m, size_, part);
     k_reduce_parts<<<m, 256>>>(part, nb, m, res);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpy(out, res, m * sizeof(double), hipMemcpyDeviceToHost));

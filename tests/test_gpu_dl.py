@@ -117,10 +117,10 @@ def test_dl_errors():
         forte_amd.DavidsonLiuSolver(0, 1)
 
 
-@pytest.mark.parametrize("size", [3, 300])
+@pytest.mark.parametrize("size", [3, 300, 1001])
 def test_dl_guess_entries(size):
     """Guesses of many entries, over the edge of a block, with indices given twice (the later value stands): exact
-    eigenvectors as guesses are converged at once, to rounding (some 1e-13 of a spectrum of at most 30)."""
+    eigenvectors as guesses are converged at once, to rounding (some 1e-13 of a spectrum of at most 100)."""
     import forte_amd
     M = synthetic(size)
     w, V = np.linalg.eigh(M)
