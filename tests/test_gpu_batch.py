@@ -58,6 +58,25 @@ def test_batch_matches_single_solver():
         assert np.abs(np.array(r["energies"]) - np.array(s.energies())).max() < 1e-9
 
 
+@pytest.mark.parametrize("nroot", [1, 3, 4])
+def test_batch_overlap_pairs(nroot):
+    """One, three and four roots: a few to more than 128 new overlaps an iteration (whole tiles a thread and parts of
+    2, 4 and 8), against one solver per problem at the same thresholds (both within e_conv of the eigenvalue)."""
+    import forte_amd
+    from forte_amd.batch import seeded_batch, solve_batch
+    sel = [p for p in seeded_batch(40) if p[0] == 8][:2]
+    opts = {"E_CONVERGENCE": 1e-11, "R_CONVERGENCE": 1e-7, "DL_MAXITER": 400, "DL_SUBSPACE_PER_ROOT": 8}
+    say("batch overlap pairs", nroot, sel)
+    res, _, _ = solve_batch(sel, nroot=nroot, options=opts)
+    for (n, seed), r in zip(sel, res):
+        s = forte_amd.FCISolver(n // 2, n // 2, 1, nroot,
+                                forte_amd.make_active_space_integrals(*forte_amd.seeded_integrals(n, seed)))
+        s.set_options(opts)
+        s.compute_energy()
+        assert r["converged"]
+        assert np.abs(np.array(r["energies"]) - np.array(s.energies())).max() < 1e-9
+
+
 def test_batch_n10_n12_members(oracle):
     """n = 10 members against full oracle solves; n = 12 (853,776 determinants, beyond a quick
     oracle solve) through oracle Slater-rules sigma rows of the batched eigenvectors (residuals),
