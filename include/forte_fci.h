@@ -206,7 +206,8 @@ int fci_sigma_device_noalloc(fci_solver* s, const void* C_dev, void* sigma_dev, 
  * eta-symmetric (not checked: for other C the result is not H C). */
 int fci_sigma_ms0_device(fci_solver* s, const void* C_dev, void* sigma_dev, int dtype, int eta, void* stream);
 /* Per-kernel device time (ms) of the last fci_sigma_device call measured with HIP events:
- * [0] same-spin beta (incl. transposes), [1] same-spin alpha, [2] alpha-beta. */
+ * [0] same-spin beta (incl. transposes), [1] same-spin alpha, [2] alpha-beta. Small spaces, whose
+ * same-spin terms are one dense product, report both under [0]. */
 int fci_sigma_timings(const fci_solver* s, double* ms3);
 /* FCISolver::form_Hdiag_det (fci_solver_initial_guess.cc:151-172), host buffer of ndet */
 int fci_hdiag(fci_solver* s, double* out);
