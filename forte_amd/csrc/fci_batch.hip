@@ -1135,7 +1135,7 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
                     DBuf<double*> dh(P);
                     dg.upload(gp.data(), P);
                     dh.upload(hp.data(), P);
-                    dense_same_batch(spin ? C.sb : C.sa, dg.p, C.gd[spin], dh.p, P, C.stream);
+                    dense_same_batch(spin ? C.sb : C.sa, dg.p, C.gd[spin], spin == 1, dh.p, P, C.stream);
                     HIPCHK(hipStreamSynchronize(C.stream));
                 }
             }

@@ -12,11 +12,13 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 #define GLOBAL_MEM __attribute__((address_space(1)))
 
 // Row I of the same-spin operator over the strings of one spin, from the pair cliques: every hole string K
-// inside I contributes s_m s_m' g'[m][m'] to column I_m'. One block per row; the members of a clique are
+// inside I contributes s_m s_m' g'[m][m'] to column I_m' (trans: row I of the operator's transpose, with
+// g'[m'][m]; one-electron integrals need not be symmetric). One block per row; the members of a clique are
 // different strings, so a thread owns each of them and the sum over K runs in a fixed order.
 __global__ __launch_bounds__(64) void k_dense_same(const uint32_t* __restrict__ clq, int M, int64_t nstr,
                                                    const uint32_t* __restrict__ own, int nown,
-                                                   const double* __restrict__ G, int gdim, double* __restrict__ H,
+                                                   const double* __restrict__ G, int gdim, bool trans,
+                                                   double* __restrict__ H,
                                                    const double* const* __restrict__ G_t = nullptr,
                                                    double* const* __restrict__ H_t = nullptr) {
     extern __shared__ double row[];  // [nstr]
@@ -31,10 +33,10 @@ __global__ __launch_bounds__(64) void k_dense_same(const uint32_t* __restrict__ 
         const uint32_t slot = own[I * nown + j];
         const uint32_t e = clq[slot];
         const uint32_t* ent = clq + size_t(slot / uint32_t(M)) * M;
-        const double* g = G + size_t((e >> 21) & 0x3FFu) * gdim;
+        const uint32_t ge = (e >> 21) & 0x3FFu;
         for (int m = threadIdx.x; m < M; m += 64) {
-            const uint32_t f = ent[m];
-            const double t = g[(f >> 21) & 0x3FFu];
+            const uint32_t f = ent[m], gf = (f >> 21) & 0x3FFu;
+            const double t = G[trans ? size_t(gf) * gdim + ge : size_t(ge) * gdim + gf];
             row[f & kAddrMask] += ((e ^ f) >> 31) ? -t : t;
         }
         __syncthreads();
@@ -44,8 +46,8 @@ __global__ __launch_bounds__(64) void k_dense_same(const uint32_t* __restrict__ 
 
 constexpr int DN_TH = 512;
 
-// S (+)= s C + Ha C + C Hb, C and S Na x Nb, Ha Na x Na, Hb Nb x Nb symmetric (null: no such term), in
-// FP64 whatever the vectors' type. Block: 32 WT x 32 WT outputs, four waves of 16 WT x 16 WT for the even k-steps and
+// S (+)= s C + Ha C + C Hb, C and S Na x Nb, Ha Na x Na the alpha operator, Hb Nb x Nb the transpose of the
+// beta operator (null: no such term), in FP64 whatever the vectors' type. Block: 32 WT x 32 WT outputs, four waves of 16 WT x 16 WT for the even k-steps and
 // four for the odd ones (two a SIMD: one's LDS reads and waits beside the other's products), k in chunks of
 // 64 / WT through two LDS buffers, the next chunk's loads in
 // flight during the products. A rows are padded
@@ -222,15 +224,15 @@ bool dense_same_use(const SpinTables& a, const SpinTables& b, size_t w) {
     return a.nstr <= most && b.nstr <= most;
 }
 
-void dense_same_device(const SpinTables& sp, const double* d_g, int gdim, double* d_h, hipStream_t st) {
+void dense_same_device(const SpinTables& sp, const double* d_g, int gdim, bool trans, double* d_h, hipStream_t st) {
     k_dense_same<<<unsigned(sp.nstr), 64, size_t(sp.nstr) * sizeof(double), st>>>(sp.clq.p, sp.M, sp.nstr, sp.own.p,
-                                                                                 sp.nown, d_g, gdim, d_h);
+                                                                                 sp.nown, d_g, gdim, trans, d_h);
     HIPCHK(hipGetLastError());
 }
-void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, double* const* h_t, int nprob,
-                      hipStream_t st) {
+void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, bool trans, double* const* h_t,
+                      int nprob, hipStream_t st) {
     k_dense_same<<<dim3(unsigned(sp.nstr), unsigned(nprob)), 64, size_t(sp.nstr) * sizeof(double), st>>>(
-        sp.clq.p, sp.M, sp.nstr, sp.own.p, sp.nown, nullptr, gdim, nullptr, g_t, h_t);
+        sp.clq.p, sp.M, sp.nstr, sp.own.p, sp.nown, nullptr, gdim, trans, nullptr, g_t, h_t);
     HIPCHK(hipGetLastError());
 }
 template <class T>

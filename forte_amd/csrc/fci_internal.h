@@ -164,8 +164,8 @@ struct DevInts {
     DBuf<float> g2f_off[2];
     DBuf<float> gdiag[2];
     int gdim[2] = {0, 0};
-    // the same-spin operators of small spaces as dense matrices (fci_dense.hip); empty where the cliques
-    // are used. hs[1] stays empty when both spins have the same one.
+    // the same-spin operators of small spaces as dense matrices (fci_dense.hip), the beta one transposed;
+    // empty where the cliques are used. hs[1] stays empty when hs[0] is the matrix of both spins.
     DBuf<double> hs[2];
     bool dense = false;
     const double* same(int spin) const { return hs[spin && hs[1].p ? 1 : 0].p; }
@@ -255,13 +255,13 @@ bool batch_sigma_supported(const SpinTables& a, const SpinTables& b, std::string
 // elements of scratch per item; *off_yt and *off_e: offsets of Y^T and E inside it (C^T at 0); dense: no E
 size_t batch_sigma_scratch_elems(const SpinTables& a, const SpinTables& b, bool dense, size_t* off_yt, size_t* off_e);
 // ---- dense same-spin operators of small spaces (fci_dense.hip) -----------------------------------
-// whether sigma with w-byte elements uses them; the operator of one spin (nstr x nstr) from its cliques,
-// for one problem and for several of one shape; S (+)= scale C + Ha C + C Hb (null: no such term), for one
-// vector and for the items of a batch
+// whether sigma with w-byte elements uses them; the operator of one spin (nstr x nstr) from its cliques, or
+// its transpose, for one problem and for several of one shape; S (+)= scale C + Ha C + C Hb with Hb the
+// transposed beta operator (null: no such term), for one vector and for the items of a batch
 bool dense_same_use(const SpinTables& a, const SpinTables& b, size_t w);
-void dense_same_device(const SpinTables& sp, const double* d_g, int gdim, double* d_h, hipStream_t st);
-void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, double* const* h_t, int nprob,
-                      hipStream_t st);
+void dense_same_device(const SpinTables& sp, const double* d_g, int gdim, bool trans, double* d_h, hipStream_t st);
+void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, bool trans, double* const* h_t,
+                      int nprob, hipStream_t st);
 template <class T>
 void dense_same_apply(const T* C, T* S, int64_t Na, int64_t Nb, const double* Ha, const double* Hb, T scale, bool add,
                       hipStream_t st);

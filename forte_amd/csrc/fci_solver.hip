@@ -419,7 +419,12 @@ class Solver {
         }
         di_.dense = dense_same_use(sa_, sb_, sizeof(double));
         if (di_.dense) {
-            const bool shared = na_ == nb_ && pk.g2[0] == pk.g2[1];
+            // one matrix for both spins: the same pair operators, and symmetric ones (the beta matrix is the transpose)
+            bool shared = na_ == nb_ && pk.g2[0] == pk.g2[1];
+            const int gd = pk.gd[0];
+            for (int i = 0; shared && i < gd; ++i)
+                for (int j = 0; j < i; ++j)
+                    shared = shared && pk.g2[0][size_t(i) * gd + j] == pk.g2[0][size_t(j) * gd + i];
             for (int spin = 0; spin < 2; ++spin) {
                 const SpinTables& sp = spin ? sb_ : sa_;
                 if (shared && spin) {
@@ -428,7 +433,7 @@ class Solver {
                 }
                 const size_t need = sp.d > 0 ? size_t(sp.nstr) * sp.nstr : 0;
                 if (di_.hs[spin].n != need) di_.hs[spin].alloc(need);
-                if (need) dense_same_device(sp, di_.g2[spin].p, di_.gdim[spin], di_.hs[spin].p, 0);
+                if (need) dense_same_device(sp, di_.g2[spin].p, di_.gdim[spin], spin == 1, di_.hs[spin].p, 0);
             }
             HIPCHK(hipStreamSynchronize(0));
         }

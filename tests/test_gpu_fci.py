@@ -170,6 +170,33 @@ def test_sigma_dense_same_spin(oracle, n, na, nb):
     assert err < 6e-7  # as test_sigma_mixed
 
 
+# One-electron operators that are not symmetric and differ between the spins (an effective Hamiltonian):
+# sigma_I = sum_J H_IJ C_J with the rows of both spins' operators. Dense same-spin matrices (one-electron and
+# pair operators, equal counts with equal and with different spin operators) and cliques (13 orbitals).
+@pytest.mark.parametrize("n,na,nb", [(5, 1, 1), (6, 3, 3), (6, 1, 3), (8, 4, 4), (9, 4, 3), (12, 2, 6), (13, 2, 6)])
+@pytest.mark.parametrize("same", [True, False])
+def test_sigma_nonsymmetric_one_electron(oracle, n, na, nb, same):
+    import forte_amd
+    say("sigma nonsymmetric", n, na, nb, same)
+    p = seeded_problem(n, na, nb, 57 + n, e_core=0.3)
+    rng = np.random.default_rng(n + nb)
+    ha = p["h"] + 0.3 * rng.standard_normal((n, n))
+    hb = ha if same else p["h"] + 0.3 * rng.standard_normal((n, n))
+    o = oracle.Oracle(n, na, nb, ha, hb, p["aa"], p["ab"], p["aa"], p["e_core"])
+    ints = forte_amd.ActiveSpaceIntegrals(n, ha, hb, p["aa"], p["ab"], p["aa"], p["e_core"])
+    g = forte_amd.FCISolver(na, nb, abs(na - nb) + 1, 1, ints)
+    C = rng.standard_normal(o.ndet)
+    C /= np.linalg.norm(C)
+    ref = o.sigma(C)
+    assert np.abs(g.sigma(C) - ref).max() < 1e-12 * max(1.0, np.abs(ref).max())
+    c32 = forte_amd.DeviceArray(o.ndet, "float32")
+    s32 = forte_amd.DeviceArray(o.ndet, "float32")
+    c32.upload(C.astype(np.float32))
+    g.sigma_arrays(c32, s32)
+    err = np.linalg.norm(s32.download().astype(np.float64) - ref) / np.linalg.norm(ref)
+    assert err < 2e-5  # BF16x3 leaves out the product of two low parts, 2^-16 of a term; a transposed operator: 1e-2
+
+
 def test_sigma_device_fp64_matches_host(oracle):
     import forte_amd
     p = seeded_problem(8, 4, 4, 5)
