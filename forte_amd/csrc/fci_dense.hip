@@ -194,14 +194,19 @@ __global__ __launch_bounds__(DN_TH) void k_dense_apply(const T* __restrict__ C, 
             }
 }
 
+size_t lds_bytes(int tl, int kc) { return size_t(2) * (tl * (kc + 2) + kc * (tl + 16)) * sizeof(double); }
+template <class K> void allow_lds(K kern, size_t sh) {
+    HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
+}
+
 template <class T>
 void launch(const T* C, T* S, int64_t Na, int64_t Nb, const double* Ha, const double* Hb, T scale, bool add, int nitem,
             const void* const* act, const T* const* C_t, T* const* S_t, const double* const* Ha_t,
             const double* const* Hb_t, hipStream_t st) {
     auto tiles = [&](int64_t t) { return ((Na + t - 1) / t) * ((Nb + t - 1) / t); };
     auto go = [&](auto kern, int tl, int kc) {
-        const size_t sh = size_t(2) * (tl * (kc + 2) + kc * (tl + 16)) * sizeof(double);
-        HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
+        const size_t sh = lds_bytes(tl, kc);
+        if (!act) allow_lds(kern, sh);  // batched launches are captured: dense_same_prepare did it
         kern<<<dim3(unsigned((Nb + tl - 1) / tl), unsigned((Na + tl - 1) / tl), unsigned(nitem)), DN_TH, sh, st>>>(
             C, S, int(Na), int(Nb), Ha, Hb, scale, add ? 1 : 0, act, C_t, S_t, Ha_t, Hb_t);
         HIPCHK(hipGetLastError());
@@ -244,6 +249,10 @@ template void dense_same_apply<double>(const double*, double*, int64_t, int64_t,
                                        bool, hipStream_t);
 template void dense_same_apply<float>(const float*, float*, int64_t, int64_t, const double*, const double*, float, bool,
                                       hipStream_t);
+void dense_same_prepare() {
+    allow_lds(k_dense_apply<double, 2>, lds_bytes(64, 32));
+    allow_lds(k_dense_apply<double, 1>, lds_bytes(32, 64));
+}
 void dense_same_apply_batch(int64_t Na, int64_t Nb, int nitem, const void* const* act, const double* const* C_t,
                             double* const* S_t, const double* const* Ha_t, const double* const* Hb_t, hipStream_t st) {
     launch<double>(nullptr, nullptr, Na, Nb, nullptr, nullptr, 0.0, false, nitem, act, C_t, S_t, Ha_t, Hb_t, st);

@@ -265,6 +265,7 @@ void dense_same_batch(const SpinTables& sp, const double* const* g_t, int gdim, 
 template <class T>
 void dense_same_apply(const T* C, T* S, int64_t Na, int64_t Nb, const double* Ha, const double* Hb, T scale, bool add,
                       hipStream_t st);
+void dense_same_prepare();  // kernel attributes of the batched form (part of batch_sigma_prepare)
 void dense_same_apply_batch(int64_t Na, int64_t Nb, int nitem, const void* const* act, const double* const* C_t,
                             double* const* S_t, const double* const* Ha_t, const double* const* Hb_t, hipStream_t st);
 

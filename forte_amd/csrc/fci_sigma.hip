@@ -2299,6 +2299,7 @@ template <int KS> static void batch_ab2_attr(const SpinTables& b) {
 }
 
 void batch_sigma_prepare(const SpinTables& a, const SpinTables& b) {
+    dense_same_prepare();
     if (ab5_f64_ok(a, b)) return ab5_f64_prepare(a, b);
     switch (ab2_f64_ks(a)) {
 #define F64CASE(K) \
