@@ -56,7 +56,8 @@ __global__ __launch_bounds__(256 * ab5m_row_waves(KS, NMT), ab5m_waves(KS, NMT))
     const float* __restrict__ C, float* __restrict__ S, int64_t Na, int64_t Nb, const uint32_t* __restrict__ into_a,
     int ns, const uint32_t* __restrict__ str_a, const uint16_t* __restrict__ outT, int ntile, int np,
     const float* __restrict__ vpk) {
-    constexpr int WM = ab5m_row_waves(KS, NMT), NT = (NMT + WM - 1) / WM, TH = 256 * WM, NW = 4;  // NW: column waves
+    constexpr int WM = ab5m_row_waves(KS, NMT), NT = (NMT + WM - 1) / WM;
+    const int TH = blockDim.x, NW = TH / (64 * WM);  // NW: column waves
     extern __shared__ __attribute__((aligned(16))) double srow[];  // [ab_row_slots(Nb)]
     __shared__ uint32_t ent[KS * 32];
     __shared__ __attribute__((aligned(16))) float vdg[NT * WM * 16];
@@ -64,7 +65,8 @@ __global__ __launch_bounds__(256 * ab5m_row_waves(KS, NMT), ab5m_waves(KS, NMT))
     if (Ja >= Na) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, cl = lane & 15;
-    const int wc = wave % NW, t0 = wave / NW * NT;  // column wave (waves w and w + 4 share a SIMD), first row tile
+    // row wave, column wave (waves w and w + 4 share a SIMD), first row tile
+    const int rw = WM == 2 && wave >= NW, wc = wave - rw * NW, t0 = rw * NT;
     for (int i = tid; i < KS * 32; i += TH) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
     for (int i = tid; i < int(ab_row_slots(Nb)); i += TH) srow[i] = 0.0;
     const uint32_t occ = str_a[Ja];
@@ -241,8 +243,11 @@ template <int KS, int NMT> void run(const Ab5mLaunch& l) {
     auto kern = k_ab5_mixed<KS, NMT>;
     const size_t sh = size_t(ab_row_slots(l.b.nstr)) * sizeof(double);
     HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
-    kern<<<xcd_grid(l.a.nstr), 256 * ab5m_row_waves(KS, NMT), sh, l.st>>>(l.C, l.S, l.a.nstr, l.b.nstr, l.a.into.p, l.a.ns, l.a.str.p,
-                                                    l.b.outT.p, l.b.npp >> 4, l.b.np, l.vpk);
+    // column waves: none without a chunk of the row (1365 rows of 15 strings, 15 orbitals: 45.4 -> 17.5 us, 42.4 in
+    // the general kernel, which took these rows before)
+    const unsigned nw = unsigned(std::min<int64_t>(4, (l.b.nstr + 31) / 32));
+    kern<<<xcd_grid(l.a.nstr), 64 * nw * ab5m_row_waves(KS, NMT), sh, l.st>>>(
+        l.C, l.S, l.a.nstr, l.b.nstr, l.a.into.p, l.a.ns, l.a.str.p, l.b.outT.p, l.b.npp >> 4, l.b.np, l.vpk);
     HIPCHK(hipGetLastError());
 }
 

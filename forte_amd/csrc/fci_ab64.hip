@@ -20,8 +20,7 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nwork) {
 }
 inline unsigned xcd_grid(int64_t nwork) { return unsigned(((nwork + 7) / 8) * 8); }
 
-constexpr int AB5_TH = 256;  // four waves
-constexpr int AB5_NW = AB5_TH / 64;
+constexpr int AB5_TH = 256;  // four waves; blocks of short rows have fewer
 
 // registers of a wave: A operands, accumulators, B operands, row offsets, targets and the rest
 constexpr int ab5_regs(int ks, int nmt) { return 2 * nmt * ks + 8 * nmt + 3 * ks + 2 * nmt + 40; }
@@ -65,12 +64,13 @@ __global__ __launch_bounds__(AB5_TH, ab5_waves(KS, NMT)) void k_ab5_f64(
     const GLOBAL_MEM double* vpkg = (const GLOBAL_MEM double*)vpk;
     const int64_t Ja = xcd_remap(blockIdx.x, Na);
     if (Ja >= Na) return;
+    const int th = blockDim.x, nw = th >> 6;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, cl = lane & 15;
-    for (int i = tid; i < KS * 4; i += AB5_TH) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
-    for (int i = tid; i < int(ab_row_slots(Nb)); i += AB5_TH) srow[i] = 0.0;
+    for (int i = tid; i < KS * 4; i += th) ent[i] = i < ns ? into_a[Ja * ns + i] : kInvalid;
+    for (int i = tid; i < int(ab_row_slots(Nb)); i += th) srow[i] = 0.0;
     const uint32_t occ = str_a[Ja];
-    for (int r = tid; r < NMT * 16; r += AB5_TH) {  // diagonal excitations: sum_{q in Ja} (qq|r)
+    for (int r = tid; r < NMT * 16; r += th) {  // diagonal excitations: sum_{q in Ja} (qq|r)
         double d = 0.0, t[16];                      // every orbital's row is read, all loads in flight
 #pragma unroll
         for (int q = 0; q < 16; ++q) t[q] = vpkg[(occ >> q) & 1u ? size_t(q * (q + 1) / 2 + q) * np + min(r, np - 1) : 0];
@@ -146,8 +146,8 @@ __global__ __launch_bounds__(AB5_TH, ab5_waves(KS, NMT)) void k_ab5_f64(
         for (int j = 0; j < NMT; ++j) load_t(j);
         // each B operand and target is replaced by the next chunk's as soon as it has been used, so the
         // loads are in flight for a whole chunk (the last chunk loads itself again)
-        for (int ch = wave; ch < nch; ch += AB5_NW) {
-            aim(ch + AB5_NW < nch ? ch + AB5_NW : ch);
+        for (int ch = wave; ch < nch; ch += nw) {
+            aim(ch + nw < nch ? ch + nw : ch);
             d4 acc[NMT];
 #pragma unroll
             for (int j = 0; j < NMT; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
@@ -176,16 +176,24 @@ __global__ __launch_bounds__(AB5_TH, ab5_waves(KS, NMT)) void k_ab5_f64(
     __syncthreads();
     GLOBAL_MEM double* Srow = (GLOBAL_MEM double*)S + Ja * Nb;
     constexpr int U = 8;
-    for (int i0 = tid; i0 < int(Nb); i0 += U * AB5_TH) {
+    for (int i0 = tid; i0 < int(Nb); i0 += U * th) {
         double s[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) s[u] = Srow[min(i0 + u * AB5_TH, int(Nb) - 1)];
+        for (int u = 0; u < U; ++u) s[u] = Srow[min(i0 + u * th, int(Nb) - 1)];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int i = i0 + u * AB5_TH;
+            const int i = i0 + u * th;
             if (i < int(Nb)) Srow[i] = s[u] + srow[ab_slot(i)];
         }
     }
+}
+
+// Waves of a block: none without a chunk of the row. Rows of at most 8 chunks get one wave once there are rows
+// for every SIMD: each wave loads all of A, and that is then most of its time. 16 orbitals, 12870 rows: 16
+// strings 642 -> 178 us (586 in the kernel before this one), 120 strings 1063 -> 641 (1032).
+unsigned block_waves(int64_t rows, int64_t nb) {
+    const int64_t nch = (nb + 15) / 16;
+    return nch <= 8 && rows >= 1024 ? 1 : unsigned(std::min<int64_t>(AB5_TH / 64, nch));
 }
 
 struct Ab5Launch {
@@ -205,7 +213,7 @@ template <int KS, int NMT> void run(const Ab5Launch& l) {
         HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(sh)));
     if (l.prepare) return;
     const unsigned ny = l.t ? unsigned(l.t->nitem) : 1;
-    kern<<<dim3(xcd_grid(l.a.nstr), ny), AB5_TH, sh, l.st>>>(
+    kern<<<dim3(xcd_grid(l.a.nstr), ny), 64 * block_waves(l.a.nstr * ny, l.b.nstr), sh, l.st>>>(
         l.C, l.S, l.a.nstr, l.b.nstr, l.a.into.p, l.a.ns, l.a.str.p, l.b.outT.p, l.b.npp >> 4, l.b.np, l.vpk,
         l.t ? l.t->act : nullptr, l.t ? l.t->c : nullptr, l.t ? l.t->s : nullptr, l.t ? l.t->vpk : nullptr);
     HIPCHK(hipGetLastError());
@@ -213,7 +221,9 @@ template <int KS, int NMT> void run(const Ab5Launch& l) {
 
 // The smallest instance with room for ns excitations and the diagonal one in its k-steps of 4; false:
 // none. Run when l is given. For every tile count (orbital count) the list holds the exact counts of
-// its half-filled spaces and a few lower ones for other fillings.
+// its half-filled spaces and a few lower ones for other fillings (14 and 16 orbitals: also that of one
+// electron or hole, whose few rows leave the chip idle; 16 rows of 12870 strings 569 -> 381 us, 500 before
+// this kernel).
 template <int NMT, int KS, int... More> bool pick(int ns, const Ab5Launch* l) {
     if (ns < 4 * KS) {
         if (l) run<KS, NMT>(*l);
@@ -231,9 +241,9 @@ bool dispatch(const SpinTables& a, const SpinTables& b, const Ab5Launch* l) {
         case 4: return pick<4, 5, 7>(ns, l);
         case 5: return pick<5, 5, 7, 8, 9, 10>(ns, l);
         case 6: return pick<6, 6, 8, 10, 11>(ns, l);
-        case 7: return pick<7, 7, 9, 11, 13>(ns, l);
+        case 7: return pick<7, 4, 7, 9, 11, 13>(ns, l);
         case 8: return pick<8, 7, 10, 13, 15>(ns, l);
-        case 9: return pick<9, 8, 11, 14, 16, 17>(ns, l);
+        case 9: return pick<9, 4, 8, 11, 14, 16, 17>(ns, l);
         default: return false;
     }
 }

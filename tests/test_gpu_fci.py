@@ -149,6 +149,20 @@ def test_sigma_mixed_chunk_edges(oracle, n, na, nb):
     assert err < (3e-6 if n >= 15 else 6e-7)
 
 
+# Blocks with fewer than four (column) waves, for rows of 1, 2 and 3 chunks (FP64: 16 columns, mixed: 32, with one
+# and two row waves) and of 8 chunks with 1024 rows and more, and the FP64 instances of one electron or hole at
+# 14 and 16 orbitals; bounds as above.
+@pytest.mark.parametrize("n,na,nb", [(8, 3, 2), (9, 3, 2), (16, 4, 1), (16, 4, 2), (16, 4, 15), (16, 1, 2), (16, 15, 3),
+                                     (14, 1, 2), (14, 13, 3)])
+def test_sigma_fp64_short_rows(oracle, n, na, nb):
+    test_sigma_fp64_chunk_edges(oracle, n, na, nb)
+
+
+@pytest.mark.parametrize("n,na,nb", [(11, 3, 2), (12, 3, 2), (14, 4, 2), (13, 5, 2), (15, 4, 1), (15, 4, 14)])
+def test_sigma_mixed_short_rows(oracle, n, na, nb):
+    test_sigma_mixed_chunk_edges(oracle, n, na, nb)
+
+
 # The dense same-spin product: ragged tiles of 32 and 64 and ragged k chunks in both products, 64 x 64
 # tiles (924 x 792), one of the two terms missing, one-electron operators.
 @pytest.mark.parametrize("n,na,nb", [(6, 0, 3), (6, 3, 0), (7, 3, 1), (9, 2, 2), (12, 2, 1), (12, 6, 1), (12, 1, 6),
