@@ -224,7 +224,12 @@ void launch(const T* C, T* S, int64_t Na, int64_t Nb, const double* Ha, const do
 // same-spin terms, dense against cliques (MI355X, FP64): 6 orbitals 7 / 26 us (4 us of them the timing
 // events), 8: 10 / 31, 10: 14 / 41, 11: 23 / 60, 12: 101 / 122, 13 (1716 x 1716): 456 / 451; FP32 at 11
 // orbitals 23 / 53 us, at 12 orbitals (in FP64 inside) 101 / 74.
+// One column and no beta term (fully polarized electrons): the cliques need no transposes, and for many strings in
+// small cliques their two launches beat a product of which a tile uses one column: 924 strings in cliques of 28 (12
+// orbitals, 6 electrons) 20.7 against 23.6 us, 792 in 21: 19.7 / 21.8, 715 in 15: 18.2 / 20.9; but 792 in 36: 24.6 /
+// 21.8, 560 in 10: 23.3 / 17.9, 495 in 15: 16.6 / 17.0.
 bool dense_same_use(const SpinTables& a, const SpinTables& b, size_t w) {
+    if (b.d == 0 && b.nstr == 1 && a.nstr > 600 && a.M <= 28) return false;
     const int64_t most = w == 8 ? 924 : 462;
     return a.nstr <= most && b.nstr <= most;
 }

@@ -211,6 +211,13 @@ def test_sigma_nonsymmetric_one_electron(oracle, n, na, nb, same):
     assert err < 2e-5  # BF16x3 leaves out the product of two low parts, 2^-16 of a term; a transposed operator: 1e-2
 
 
+# A single column without a beta term: dense up to 600 strings or cliques of more than 28 members (715 strings in 55,
+# 495 in 15), otherwise the cliques (715 strings in 15, 792 in 21).
+@pytest.mark.parametrize("n,na", [(13, 4), (12, 8), (13, 9), (12, 7)])
+def test_sigma_one_column(oracle, n, na):
+    test_sigma_dense_same_spin(oracle, n, na, 0)
+
+
 def test_sigma_device_fp64_matches_host(oracle):
     import forte_amd
     p = seeded_problem(8, 4, 4, 5)
