@@ -1580,8 +1580,11 @@ int fci_rdms(fci_solver* s, int rl, int rr, int level, double* g1a, double* g1b,
         // with the alpha-beta 2-RDM at hand the 1-RDMs are its partial traces, sum_r <E^alpha_pq E^beta_rr> =
         // nb <E^alpha_pq>; otherwise from the vectors
         const bool traced = level >= 2 && S.na_ > 0 && S.nb_ > 0;
+        // (released with the buffers of the 2-RDM: a hipFree in between waits a second time, 8 us a call)
+        fci::DBuf<double> d1a, d1b;
         if (!traced) {
-            fci::DBuf<double> d1a(n2), d1b(n2);
+            d1a.alloc(n2);
+            d1b.alloc(n2);
             fci::rdm1_device(S.sa_, S.sb_, L, R, d1a.p, d1b.p, 0);
             HIPCHK(hipStreamSynchronize(0));
             if (g1a) d1a.download(g1a, n2);
