@@ -588,7 +588,8 @@ __global__ void k_csf_hdiag(const double* __restrict__ hd, double* __restrict__ 
 // The same with the configuration's determinant diagonals staged in LDS: block (x, y) covers `cpb` configurations
 // and CSF rows [y rpb, y rpb + rpb), a row per wave (its nonzeros over the lanes) or per thread, so the addresses
 // are formed once per block and no sum is a chain of dependent loads. The six open-shell classes of 12 orbitals with 7 + 5
-// electrons, triplet: 1.53 -> 0.10 ms; the kernel above stays for rows past the LDS (17 open shells and more).
+// electrons, triplet: 1.53 -> 0.10 ms; the kernel above stays for rows past the LDS (17 open
+// shells and more) and for fci_hdiag_csf_unstaged.
 __global__ __launch_bounds__(256) void k_csf_hdiag_lds(const double* __restrict__ hd, double* __restrict__ out,
                                                        const uint32_t* __restrict__ docc,
                                                        const uint32_t* __restrict__ socc,
@@ -959,11 +960,11 @@ template <class TO> void CsfSpace::to_det(const double* csf, TO* det, int64_t nd
     HIPCHK(hipGetLastError());
 }
 
-void CsfSpace::hdiag(const double* hdet, double* hcsf, hipStream_t st) const {
+void CsfSpace::hdiag(const double* hdet, double* hcsf, hipStream_t st, bool staged) const {
     for (const auto& C : cls_) {
         if (C.nconf == 0 || C.ncsf == 0) continue;
         const size_t row_bytes = size_t(C.ndp) * sizeof(double);
-        if (row_bytes <= kCsfLdsBytes) {
+        if (staged && row_bytes <= kCsfLdsBytes) {
             // configurations up to 32 KB a block (at least one) as long as that leaves 1024 blocks; below that
             // their rows are split over blocks, 16 at least
             const int64_t fit = int64_t(std::max<size_t>(1, std::min<size_t>(64, (32u << 10) / row_bytes)));

@@ -372,7 +372,8 @@ class CsfSpace {
     // csf_C_to_det_C (ci_spin_adaptation.cc:106-121); determinants outside the CSFs are zeroed
     template <class TO> void to_det(const double* csf, TO* det, int64_t ndet, hipStream_t st) const;
     // sum_j c_j^2 H_jj per CSF
-    void hdiag(const double* hdet, double* hcsf, hipStream_t st) const;
+    // staged: determinant rows that fit are staged in LDS; else every diagonal is read from memory
+    void hdiag(const double* hdet, double* hcsf, hipStream_t st, bool staged = true) const;
     // host walk over every CSF: (CSF index, its determinants with coefficients)
     void for_each_csf(const std::function<void(int64_t, const std::vector<std::pair<Det, double>>&)>& f) const;
 

@@ -600,7 +600,7 @@ class Solver {
         return *csf_;
     }
     // FCISolver::form_Hdiag_csf (fci_solver_initial_guess.cc:111-149) into csf_hd_
-    void compute_hdiag_csf();
+    void compute_hdiag_csf(bool staged = true);
     // eigenvector `root` in the determinant basis (device); spin-adapted solves convert theirs
     const double* evec_device(int root) const {
         if (csf_solved_) return csf_ev_.p + size_t(root) * ndet_;
@@ -806,11 +806,11 @@ struct LPRun {
     }
 };
 
-void Solver::compute_hdiag_csf() {
+void Solver::compute_hdiag_csf(bool staged) {
     CsfSpace& cs = csf_space();
     if (csf_hd_.n < size_t(cs.ncsf())) csf_hd_.alloc(cs.ncsf());
     if (!opt_.spin_adapt_full_preconditioner) {
-        cs.hdiag(hdiag_.p, csf_hd_.p, 0);
+        cs.hdiag(hdiag_.p, csf_hd_.p, 0, staged);
         HIPCHK(hipStreamSynchronize(0));
         return;
     }
@@ -1393,16 +1393,18 @@ int fci_csf_to_det(fci_solver* s, const double* csf, double* det) {
     });
 }
 
-int fci_hdiag_csf(fci_solver* s, double* out) {
+static int hdiag_csf(fci_solver* s, double* out, bool staged) {
     if (!s || !out) return FCI_ERR_ARG;
     return guarded(&s->err, [&] {
         auto& S = *s->s;
         if (!S.have_ints_) throw Error(FCI_ERR_STATE, "integrals have not been set");
         S.compute_hdiag();
-        S.compute_hdiag_csf();
+        S.compute_hdiag_csf(staged);
         S.csf_hd_.download(out, S.csf_space().ncsf());
     });
 }
+int fci_hdiag_csf(fci_solver* s, double* out) { return hdiag_csf(s, out, true); }
+int fci_hdiag_csf_unstaged(fci_solver* s, double* out) { return hdiag_csf(s, out, false); }
 
 int64_t fci_ndet(const fci_solver* s) { return s ? s->s->ndet_ : -1; }
 int64_t fci_nstr(const fci_solver* s, int spin) { return s ? (spin ? s->s->sb_.nstr : s->s->sa_.nstr) : -1; }

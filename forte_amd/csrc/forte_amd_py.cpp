@@ -349,9 +349,9 @@ class FCISolver {
         check(fci_csf_to_det(h_, csf.data(), out.mutable_data()), fci_last_error(h_));
         return out;
     }
-    py::array_t<double> hdiag_csf() {
+    py::array_t<double> hdiag_csf(bool staged) {
         py::array_t<double> out(ncsf());
-        check(fci_hdiag_csf(h_, out.mutable_data()), fci_last_error(h_));
+        check((staged ? fci_hdiag_csf : fci_hdiag_csf_unstaged)(h_, out.mutable_data()), fci_last_error(h_));
         return out;
     }
     py::array_t<double> evec_csf(int root) {
@@ -710,7 +710,7 @@ PYBIND11_MODULE(_forte_amd, m) {
         .def("ncsf", &FCISolver::ncsf)
         .def("det_to_csf", &FCISolver::det_to_csf)
         .def("csf_to_det", &FCISolver::csf_to_det)
-        .def("hdiag_csf", &FCISolver::hdiag_csf)
+        .def("hdiag_csf", &FCISolver::hdiag_csf, py::arg("staged") = true)
         .def("evec_csf", &FCISolver::evec_csf)
         .def("ndet", &FCISolver::ndet)
         .def("nstr", &FCISolver::nstr)

@@ -175,6 +175,9 @@ int fci_csf_to_det(fci_solver* s, const double* csf, double* det);
 /* FCISolver::form_Hdiag_csf (fci_solver_initial_guess.cc:111-149), honouring
  * spin_adapt_full_preconditioner; ncsf doubles */
 int fci_hdiag_csf(fci_solver* s, double* out);
+/* the same (without the full preconditioner) for every class through the kernel that classes of 17 and more open
+ * shells take, whose determinant rows do not fit in LDS: for comparison */
+int fci_hdiag_csf_unstaged(fci_solver* s, double* out);
 /* FCISolver::evecs() row `root` of a spin-adapted solve: the eigenvector in the CSF basis */
 int fci_evec_csf(const fci_solver* s, int root, double* out);
 

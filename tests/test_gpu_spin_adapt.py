@@ -85,6 +85,18 @@ def test_hdiag_many_open_shells(oracle, n, na, nb, twoS):
     assert np.abs(s.hdiag_csf() - ref.hdiag(o.hdiag())).max() < 1e-11
 
 
+@pytest.mark.parametrize("n,na,nb,twoS", [(6, 3, 3, 0), (9, 5, 4, 1), (10, 5, 5, 2), (18, 3, 2, 1)])
+def test_hdiag_unstaged(n, na, nb, twoS):
+    """The kernel of classes whose determinant rows pass the LDS (17 open shells, 4e8 determinants and more) on small
+    classes, with byte-table ranks and with ranks summed by electron, against the staged one (checked above): sums of
+    weights adding up to 1 of diagonals of order 10, in another order; 1e-11 is 10^3 eps of that."""
+    say(f"csf diagonal unstaged n={n} na={na} nb={nb} 2S={twoS}")
+    s = solver(seeded_problem(n, na, nb, 15), 1, twoS + 1, None, 0)
+    got = s.hdiag_csf(staged=False)
+    assert np.abs(got).max() > 0.1
+    assert np.abs(got - s.hdiag_csf()).max() < 1e-11
+
+
 @pytest.mark.parametrize("n,na,nb,twoS", [(18, 2, 2, 0), (17, 3, 1, 2), (18, 3, 2, 1)])
 def test_transforms_beyond_16_orbitals_vs_oracle(n, na, nb, twoS):
     """Above 16 orbitals the string ranks are summed electron by electron (the byte tables cover
