@@ -115,6 +115,25 @@ def test_batch_n10_n12_members(oracle):
             assert abs(o.spin2(c)) < 1e-6
 
 
+@pytest.mark.parametrize("n,na,nb,mult,count", [(13, 11, 6, 6, 3), (13, 6, 6, 1, 1)])
+def test_batch_clique_classes(n, na, nb, mult, count):
+    """More than 924 strings of one spin: the same-spin terms of a class through the batched cliques, with both spins
+    (13, 11, 6) and in the spin-flip-symmetric form (13, 6, 6), against one solver per problem at the same thresholds
+    (both within e_conv of the eigenvalue)."""
+    import forte_amd
+    from forte_amd.batch import solve_many
+    say("batch cliques", n, na, nb)
+    opts = {"E_CONVERGENCE": 1e-10, "R_CONVERGENCE": 1e-6, "DL_MAXITER": 400}
+    ints = [forte_amd.make_active_space_integrals(*forte_amd.seeded_integrals(n, s)) for s in range(3, 3 + count)]
+    out = solve_many(ints, [na] * count, [nb] * count, multiplicity=mult, options=opts)
+    for i, e, ok in zip(ints, out["energies"], out["converged"]):
+        s = forte_amd.FCISolver(na, nb, mult, 1, i)
+        s.set_options(opts)
+        s.compute_energy()
+        assert ok
+        assert abs(e[0] - s.energies()[0]) < 1e-9
+
+
 def test_batch_rejects_unsupported_options():
     import forte_amd
     h, eri = forte_amd.seeded_integrals(6, 1)

@@ -59,11 +59,11 @@ def test_hdiag_bit_exact(oracle, n, na, nb):
 SIGMA_CASES = [(2, 1, 1), (3, 2, 1), (4, 2, 2), (4, 3, 2), (5, 1, 1), (6, 3, 3), (6, 2, 4), (6, 5, 1),
                (4, 4, 0), (4, 0, 4), (6, 6, 6), (7, 1, 6), (8, 4, 4), (8, 3, 5), (9, 2, 2), (10, 5, 5),
                (10, 2, 8), (12, 6, 6), (12, 4, 7),
-               # 14 to 18 orbitals: 7, 9, 10 and 11 row tiles of pairs, the alpha-beta layouts of CAS(14,14)
-               # to CAS(18,18) (few electrons keep the oracle fast)
+               # 14 to 18 orbitals: 7, 9, 10 and 11 row tiles of pairs (few electrons keep the oracle fast);
+               # 17 and up take the alpha-beta kernels behind fci_ab64.hip's
                (14, 3, 3), (16, 2, 2), (16, 3, 3), (17, 2, 2), (18, 3, 3),
-               # the alpha-beta instances the CAS(16,16) and CAS(14,14) solves run (55 and 49 alpha
-               # single excitations: 16 k-steps, 9 and 7 row tiles, the shared last row tile at 9)
+               # 55 and 49 alpha single excitations (14 and 13 k-steps) in 9 and 7 row tiles, the latter the
+               # instance of CAS(14,14); CAS(16,16)'s has 17 k-steps (test_sigma_fp64_instances)
                (16, 5, 1), (14, 7, 1), (16, 1, 5)]
 
 
@@ -99,10 +99,10 @@ def test_sigma_fp64_chunk_edges(oracle, n, na, nb):
 
 @pytest.mark.parametrize("n,na,nb", [(6, 3, 3), (8, 4, 4), (10, 5, 5), (12, 6, 6), (9, 3, 5), (14, 3, 3), (16, 2, 2),
                                      (16, 3, 3), (17, 2, 2), (18, 3, 3),
-                                     # same-spin cliques of 36, 45 and 55 members (the alpha side,
-                                     # even row length): the static-size pass-1 kernels
+                                     # (12, 4, 5): same-spin cliques of 45 members (the alpha side, even row
+                                     # length), a static-size pass-1 kernel; the others take the dense product
                                      (9, 2, 2), (10, 2, 3), (12, 4, 5), (12, 3, 2),
-                                     # 6 row tiles (n = 13) and the production k-step counts
+                                     # 6 row tiles (n = 13) and many excitations in 9 and 7 row tiles
                                      (13, 3, 3), (16, 5, 1), (14, 7, 1)])
 def test_sigma_mixed(oracle, n, na, nb):
     import forte_amd
@@ -125,6 +125,34 @@ def test_sigma_mixed(oracle, n, na, nb):
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     say("  relative error", err)
     assert err < (3e-6 if n >= 16 else 6e-7)
+
+
+# Every FP64 alpha-beta instance of 12 to 16 orbitals (k-steps of 4 excitations, row tiles of 16 pairs) that the
+# cases above leave out, one beta electron keeping the oracle fast: 12 orbitals 7; 13: 8 and 11; 14: 7, 11;
+# 15: 13, 15; 16: 11, 16, 17. And their last column chunks behind full ones (two beta electrons).
+@pytest.mark.parametrize("n,na,nb", [(12, 3, 1), (13, 3, 1), (13, 7, 1), (14, 2, 1), (14, 4, 1), (15, 5, 1), (15, 7, 1),
+                                     (16, 3, 1), (16, 7, 1), (16, 8, 1), (13, 5, 2), (15, 4, 2)])
+def test_sigma_fp64_instances(oracle, n, na, nb):
+    say("sigma fp64 instances", n, na, nb)
+    p = seeded_problem(n, na, nb, 27 + n, e_core=-0.4)
+    g, o = gpu_solver(p), cpu_oracle(oracle, p)
+    rng = np.random.default_rng(n * 10 + nb)
+    C = rng.standard_normal(o.ndet)
+    rows = rng.choice(o.ndet, size=min(o.ndet, 3000), replace=False)  # Slater rules, row by row
+    ref = o.sigma_rows(C, rows)
+    assert np.abs(g.sigma(C)[rows] - ref).max() < 1e-12 * max(1.0, np.abs(ref).max())
+
+
+# The same-spin cliques of more than 924 strings (FP64; mixed: 462) in rows of odd and of even length: FP64 cliques of
+# 55, 21, 45 and 36 members, mixed the static-size kernels of 36 (alpha side) and 55 (beta side) members.
+@pytest.mark.parametrize("n,na,nb", [(14, 5, 2), (14, 9, 2), (13, 5, 1), (13, 6, 1)])
+def test_sigma_fp64_cliques_odd_rows(oracle, n, na, nb):
+    test_sigma_fp64_chunk_edges(oracle, n, na, nb)
+
+
+@pytest.mark.parametrize("n,na,nb", [(12, 5, 3), (14, 5, 2)])
+def test_sigma_mixed_cliques(oracle, n, na, nb):
+    test_sigma_mixed(oracle, n, na, nb)
 
 
 # The mixed alpha-beta kernel at the edges of its 32-column chunks, for odd rows (the last column is read
@@ -427,7 +455,7 @@ def test_mixed_precision_solve(oracle):
 
 def test_mixed_precision_solve_cas14():
     """CAS(14,14), 11.8 million determinants: the production kernels at scale (alpha-beta with the
-    A operand in LDS, same-spin pass 1 with a compile-time clique size of 36 and staged stores).
+    A operand in registers, same-spin pass 1 with a compile-time clique size of 36 and staged stores).
     The mixed solve and its FP64 refinement must land on the FP64 energy."""
     import forte_amd
     say("mixed solve CAS(14,14)")
@@ -546,6 +574,23 @@ def test_rdms_large_cliques(oracle, n, na, nb):
     for name, a, b in zip(("g1a", "g1b", "g2aa", "g2ab", "g2bb"), [rd.g1a(), rd.g1b(), rd.g2aa(), rd.g2ab(), rd.g2bb()],
                           ref):
         assert np.abs(a - b).max() < 1e-12, name
+
+
+# 17 and 18 orbitals: the alpha-beta product of up to 16 and up to 24 tiles a wave and the one without MFMA; one beta
+# string (all orbitals filled) at up to 16 orbitals, with single columns in the alpha cliques.
+@pytest.mark.parametrize("n,na,nb", [(17, 2, 2), (17, 3, 1), (18, 3, 2), (18, 2, 3), (18, 5, 1), (6, 3, 6), (8, 4, 8), (14, 3, 14)])
+def test_rdms_general_kernels(oracle, n, na, nb):
+    say("rdms general", n, na, nb)
+    p = seeded_problem(n, na, nb, 43)
+    g, o = gpu_solver(p, 2, abs(na - nb) + 1), cpu_oracle(oracle, p)
+    g.set_die_if_not_converged(False)  # any two vectors do
+    g.set_maxiter(5)
+    g.compute_energy()
+    for (l, r) in [(0, 0), (0, 1)]:  # the bound of test_rdms_tile_edges
+        rd = g.rdms([(l, r)], 2)[0]
+        ref = o.rdms(g.evec(l), g.evec(r))
+        for a, b in zip([rd.g1a(), rd.g1b(), rd.g2aa(), rd.g2ab(), rd.g2bb()], ref):
+            assert np.abs(a - b).max() < 1e-12, (l, r)
 
 
 @pytest.mark.parametrize("n,na,nb", [(19, 2, 2), (19, 3, 2)])

@@ -92,6 +92,19 @@ def test_noalloc_sigma_matches_allocating_sigma(dtype):
         L.fci_destroy(hnd)
 
 
+@pytest.mark.parametrize("n,na,nb", [(13, 6, 2), (12, 2, 6)])
+def test_noalloc_sigma_other_routes(n, na, nb):
+    """FP64 above 924 strings, whose clique intermediates live in the scratch, and a dense one with long beta rows;
+    bounds as above."""
+    L = _lib()
+    say(f"noalloc sigma n={n} na={na} nb={nb}")
+    hnd = _create(L, n, na, nb, 4)
+    C = np.random.default_rng(4).standard_normal(L.fci_ndet(hnd))
+    ref, got = _sigma_pair(L, hnd, C, 0)
+    assert np.abs(got - ref).max() / np.abs(ref).max() < 1e-13
+    L.fci_destroy(hnd)
+
+
 def test_noalloc_refuses_problems_beyond_the_scratch():
     L = _lib()
     say("noalloc size limit: CAS(14,14)")
