@@ -1117,7 +1117,7 @@ int fci_batch_solve(int nprob, const int* norb, const int* nalpha, const int* nb
             C.g2a.alloc(g2a_h.size()); C.g2a.upload(g2a_h.data(), g2a_h.size());
             C.g2b.alloc(g2b_h.size()); C.g2b.upload(g2b_h.data(), g2b_h.size());
             // small spaces: the dense same-spin operators of every problem (the symmetric form has no
-            // beta term), unless they would take more memory than a few classes' vectors
+            // beta term), while those of the class fit in 16 GB
             const size_t ha2 = size_t(C.sa.nstr) * C.sa.nstr, hb2 = C.eta ? 0 : size_t(C.sb.nstr) * C.sb.nstr;
             C.dense = dense_same_use(C.sa, C.sb, sizeof(double)) && size_t(P) * (ha2 + hb2) * 8 <= (size_t(16) << 30);
             if (C.dense) {

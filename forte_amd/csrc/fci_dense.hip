@@ -50,8 +50,8 @@ constexpr int DN_TH = 512;
 // beta operator (null: no such term), in FP64 whatever the vectors' type. Block: 32 WT x 32 WT outputs, four waves of 16 WT x 16 WT for the even k-steps and
 // four for the odd ones (two a SIMD: one's LDS reads and waits beside the other's products), k in chunks of
 // 64 / WT through two LDS buffers, the next chunk's loads in
-// flight during the products. A rows are padded
-// to 18 and B rows to 16 more than the tile, so that the half waves' operand reads hit 64 banks.
+// flight during the products. A rows are padded by 2 doubles (to 34 and 66) and B rows by 16 (to 80 and 48), so
+// that the half waves' operand reads hit 64 banks.
 template <class T, int WT>
 __global__ __launch_bounds__(DN_TH) void k_dense_apply(const T* __restrict__ C, T* __restrict__ S, int Na, int Nb,
                                                      const double* __restrict__ Ha, const double* __restrict__ Hb,

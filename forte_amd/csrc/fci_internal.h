@@ -269,8 +269,8 @@ void dense_same_prepare();  // kernel attributes of the batched form (part of ba
 void dense_same_apply_batch(int64_t Na, int64_t Nb, int nitem, const void* const* act, const double* const* C_t,
                             double* const* S_t, const double* const* Ha_t, const double* const* Hb_t, hipStream_t st);
 
-// the FP64 alpha-beta term with the gathered rows staged in LDS (fci_ab64.hip): whether it takes these
-// tables, sigma += H_ab C with the packed integrals vpk, the batched form and its kernel attributes
+// the FP64 alpha-beta term of up to 16 orbitals (fci_ab64.hip): whether it takes these tables, sigma += H_ab C
+// with the packed integrals vpk, the batched form and its kernel attributes
 bool ab5_f64_ok(const SpinTables& a, const SpinTables& b);
 void ab5_f64(const double* C, double* S, const SpinTables& a, const SpinTables& b, const double* vpk, hipStream_t st);
 void ab5_f64_batch(const SpinTables& a, const SpinTables& b, const BatchSigmaTabs& t, hipStream_t st);

@@ -92,7 +92,9 @@ __global__ __launch_bounds__(256) void k_rdm2_targets(const uint32_t* __restrict
 // Bound by the FP64 matrix unit (64 cycles an instruction). CAS(14,14), 3432 x 3432: 3.35 ms with L = R (7 pair
 // tiles, 1.7e11 operations, 51 TFLOP/s; the tile that one wave of four lacks costs an eighth) and 6.19 ms with two vectors
 // (13 tiles, 51 TFLOP/s), where k_rdm2_ab_mfma, which stages both operands and takes the symmetric pairs of
-// both directions, took 21.8 ms; so that one is left to 17 orbitals and up.
+// both directions, took 21.8 ms. CAS(16,16): 100 ms with L = R, and 452 ms with two vectors, whose sums do not fit
+// the registers beside the rest (<5, 4>: 672 bytes of scratch a lane), against 757 for k_rdm2_ab_mfma either way;
+// so that one is left to 17 orbitals and up.
 template <int ET, int ZW>
 __global__ __launch_bounds__(R2_TH, (ET * ZW <= 16 ? 2 : 1)) void k_rdm2_ab5(
     const double* __restrict__ L, const double* __restrict__ R, int64_t Na, int64_t Nb, const uint32_t* __restrict__ into_a,

@@ -2157,8 +2157,8 @@ static bool ab2_ok(const SpinTables& a, const SpinTables& b, size_t w) {
            size_t(ab_row_slots(b.nstr)) * w <= 150 * 1024;
 }
 
-// The FP64 kernel without LDS staging takes what fci_ab64.hip's cannot hold beside a row of 15.8 to
-// 19.2 thousand strings (18 orbitals with 6 or 12 beta electrons): 9 to 12 row tiles
+// The FP64 kernel of 17 to 19 orbitals (10 to 12 row tiles), even rows of at most 19,072 strings: fci_ab64.hip's
+// holds all of A in one wave's registers, which ends at 16 orbitals, and takes every space up to there
 static bool ab2_f64_ok(const SpinTables& a, const SpinTables& b) {
     return ab2_ok(a, b, sizeof(double)) && (b.np + 15) / 16 > 8;
 }
