@@ -1,6 +1,7 @@
 // fci_ab32.hip -- the mixed-precision alpha-beta term of sigma (H2_aabb,
 // fci_vector_hamiltonian.cc:194-272): FP32 vectors, BF16x3 products on v_mfma_f32_16x16x32_bf16 with
 // FP32 accumulation; per alpha row gather -> MFMA -> LDS scatter, every wave on its own columns.
+#include "fci_device.h"
 #include "fci_internal.h"
 
 #include <algorithm>
@@ -14,18 +15,6 @@ typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 // two floats at 4-byte alignment: one 8-byte load whatever the parity of the row length
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
-#define GLOBAL_MEM __attribute__((address_space(1)))
-
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nwork) {
-    const int64_t per = (nwork + 7) / 8;
-    return (b % 8) * per + b / 8;
-}
-inline unsigned xcd_grid(int64_t nwork) { return unsigned(((nwork + 7) / 8) * 8); }
-
-__device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo) {
-    hi = __bf16(x);
-    lo = __bf16(x - float(hi));
-}
 
 // Registers of a wave with all row tiles: A operands, diagonal rows and targets per tile, the raw and the
 // split columns. Where they pass 256, two waves share the row tiles of their columns (WM = 2, two waves a

@@ -1,5 +1,6 @@
 // fci_ab64.hip -- the FP64 alpha-beta term of sigma (H2_aabb, fci_vector_hamiltonian.cc:194-272) on
 // v_mfma_f64_16x16x4_f64: per alpha row gather -> MFMA -> LDS scatter, every wave on its own columns.
+#include "fci_device.h"
 #include "fci_internal.h"
 
 #include <algorithm>
@@ -10,15 +11,6 @@ namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
-// global-memory pointers, said so: a pointer picked from an item table is otherwise taken as flat, and
-// a flat load waits with the LDS counter
-#define GLOBAL_MEM __attribute__((address_space(1)))
-
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nwork) {
-    const int64_t per = (nwork + 7) / 8;
-    return (b % 8) * per + b / 8;
-}
-inline unsigned xcd_grid(int64_t nwork) { return unsigned(((nwork + 7) / 8) * 8); }
 
 constexpr int AB5_TH = 256;  // four waves; blocks of short rows have fewer
 

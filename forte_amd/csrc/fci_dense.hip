@@ -1,5 +1,6 @@
 // fci_dense.hip -- the same-spin terms of sigma for small string spaces (H0, H1 and H2_aaaa / H2_bbbb,
 // fci_vector_hamiltonian.cc:84-192) as one dense product per spin: S = s C + Haa C + C Hbb.
+#include "fci_device.h"
 #include "fci_internal.h"
 
 #include <algorithm>
@@ -9,7 +10,6 @@ namespace fci {
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-#define GLOBAL_MEM __attribute__((address_space(1)))
 
 // Row I of the same-spin operator over the strings of one spin, from the pair cliques: every hole string K
 // inside I contributes s_m s_m' g'[m][m'] to column I_m' (trans: row I of the operator's transpose, with

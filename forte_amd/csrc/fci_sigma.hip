@@ -19,6 +19,7 @@
 //
 // FP64: v_mfma_f64_16x16x4_f64. Mixed: FP32 storage, BF16x3 split products
 // (hi*hi + hi*lo + lo*hi) on v_mfma_f32_16x16x32_bf16, FP32 accumulation.
+#include "fci_device.h"
 #include "fci_internal.h"
 
 #include <algorithm>
@@ -33,13 +34,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 static inline unsigned nblk(int64_t n, int bs) { return unsigned((n + bs - 1) / bs); }
-
-// Hardware dispatches workgroup b to XCD (b % 8); give each XCD a contiguous range of work.
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t nwork) {
-    int64_t per = (nwork + 7) / 8;
-    return (b % 8) * per + b / 8;
-}
-static inline unsigned xcd_grid(int64_t nwork) { return unsigned(((nwork + 7) / 8) * 8); }
 
 // ---- elementwise helpers ---------------------------------------------------------------------
 template <class T> __global__ void k_fill(T* p, int64_t n, T v) {
@@ -411,11 +405,6 @@ __global__ __launch_bounds__(256) void k_clique_f64(const double* __restrict__ X
                 atomicAdd(&Y[int64_t(e & kAddrMask) * L + col], val);
             }
         }
-}
-
-__device__ __forceinline__ void split_bf16(float x, __bf16& hi, __bf16& lo) {
-    hi = __bf16(x);
-    lo = __bf16(x - float(hi));
 }
 
 // Mixed: FP32 storage, BF16x3 products, FP32 accumulation.
